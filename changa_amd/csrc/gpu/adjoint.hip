@@ -68,7 +68,7 @@ __device__ __forceinline__ D2 drsq(D2 a) {
 }
 
 // (da/dr) w for the hexadecapole acceleration of a staged record (the
-// formula of pc_interact, evaluated on dual numbers with tangent w).
+// formula of pc_eval, evaluated on dual numbers with tangent w).
 __device__ __forceinline__ void pc_tidal(const float4* rec, float rx, float ry, float rz, float wx,
                                          float wy, float wz, float& tx, float& ty, float& tz) {
   const D2 X = {rx, wx}, Y = {ry, wy}, Z = {rz, wz};

@@ -91,17 +91,16 @@ __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane
 // exhausted. Each wave visits the 8 queues once, starting at its own XCD's,
 // and stays on a queue until a claim comes back past its end, so every wave
 // exits after finitely many claims and no wave waits on another.
-// Three wavefronts per SIMD: up to 168 VGPRs for the three-targets-per-lane
-// loops (measured faster on the 2^22 halos than one target per lane at four
-// wavefronts). With KMAX 1 the kernel holds one chunk loop instead of three
-// and needs 139-160 VGPRs, without spills; on a sparse rung (one to three
-// targets in most buckets) it measured 16% faster than KMAX 3, on the dense
-// halos 7% slower. With KMAX 1 and cell records it is built for four
-// wavefronts (128 VGPRs: the 32-cell tile spills 2, the 64-cell tile 23),
-// which the sparse rung prefers.
+// Four wavefronts per SIMD (128 VGPRs), because the FP32 VALU issues the
+// force loops faster with four than with three (gravity_body.h: pc_cells).
+// KMAX 1 holds one chunk loop and does not spill: on a sparse rung (one to
+// three targets in most buckets), where a tile's own work weighs most, it
+// measured 7.69 ms against 11.6 for KMAX 3, whose three-targets loop spills
+// 28 to 42 registers around the tiles; on the dense 2^22 halos, where the
+// shared LDS reads weigh more, KMAX 3 measured 9.13 ms against 9.92.
 template <bool PRECISE, int KIND, int PCT, int PPT, int KMAX, bool REC>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(KMAX == 1 && REC ? 4 : 3))) void batch_kernel(BatchArgs a) {
+__attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(BatchArgs a) {
   __shared__ float4 lds[BatchLds<PCT, PPT>::f4];
   const int lane = threadIdx.x;
   const int* qbeg = a.queue;

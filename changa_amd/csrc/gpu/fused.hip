@@ -23,9 +23,7 @@
 
 namespace cgpu {
 
-constexpr int kFusedPcTile = 64;
-constexpr int kFusedRecTile = 32;  // cell tile with the 128-byte records (their prefetch fits
-                                   // the four-wavefront register budget)
+constexpr int kFusedPcTile = 64;  // cells (32 with records: 128^3 box 3.49 ms, 64: 3.35)
 constexpr int kFusedPpTile = 256;
 constexpr int kFusedRanges = kNumXcd;
 constexpr int kFusedCounterStride = 32;
@@ -86,9 +84,9 @@ __device__ bool fused_walk(const FusedArgs& a, int b, int lane, unsigned* stack,
   return ok;
 }
 
-// Four wavefronts per SIMD (128 VGPRs, a few spills outside the force loops)
-// measured 11-12% faster than the three that 141 VGPRs allow: the walk's load
-// latency is hidden behind more resident wavefronts.
+// Four wavefronts per SIMD (128 VGPRs, no spills): the walk's load latency is
+// hidden behind more resident wavefronts and the force loops' FP32
+// instructions issue together (gravity_body.h: pc_cells).
 // REC: cells from the 128-byte cell records (a.pc.cellRecords), whole-line
 // fetches in tiles of PCT.
 template <int PCT, int PPT, bool REC>
@@ -129,7 +127,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void fu
     bucket_centre<true>(a.pc.tpos64, bstart, n, cx0, cy0, cz0);
     for (int t0 = 0; t0 < n; t0 += kWave) {
       // one target per lane: the walk's stack and scratch leave no registers
-      // for more
+      // for more (two per lane: 30 spills, 2^22 halos 10.8 ms against 11.4 but
+      // 128^3 box 3.51 against 3.35 and its 256^3 rung 18.1 against 15.0)
       const Lanes l = lanes_for<1>(lane, min(kWave, n - t0));
       Target t[1];
       load_targets<true, 1>(a.pc, bstart + t0, l, cx0, cy0, cz0, t);
@@ -153,7 +152,7 @@ __global__ void fused_reset_kernel(int* counters) {
 using FusedFn = void (*)(FusedArgs);
 
 static FusedFn fused_fn(bool rec) {
-  return rec ? fused_kernel<kFusedRecTile, kFusedPpTile, true>
+  return rec ? fused_kernel<kFusedPcTile, kFusedPpTile, true>
              : fused_kernel<kFusedPcTile, kFusedPpTile, false>;
 }
 

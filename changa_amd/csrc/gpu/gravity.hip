@@ -11,16 +11,16 @@ namespace cgpu {
 // Per-bucket particle-cell kernel: one 64-lane workgroup per bucket, buckets
 // mapped to XCDs in contiguous ranges (xcd_bucket).
 // ---------------------------------------------------------------------------
-// REC: cells from the 128-byte cell records in tiles of 32 (their prefetch
-// then fits three wavefronts per SIMD), else from the wire moments in tiles
-// of kPcTile.
+// REC: cells from the 128-byte cell records, else from the wire moments; in
+// tiles of 64 either way (records in tiles of 32: 128^3 box 2.34 ms against
+// 2.22, 256^3 box with a 10% rung 8.05 against 6.11). At most two targets
+// per lane: no spills at four wavefronts per SIMD.
 template <bool PRECISE, bool REC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void pc_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pc_kernel(
     ChangaGravityLaunch a) {
-  constexpr int TILE = REC ? 32 : kPcTile;
   // staged tile; reused for the slot reduction at the end of each chunk
   __shared__ float4 rec4[(kPcTile + 1) * (kFwdRec / 4)];
-  static_assert(sizeof(rec4) >= reduce_bytes<3>(), "reduction");
+  static_assert(sizeof(rec4) >= reduce_bytes<2>(), "reduction");
 
   const int lane = threadIdx.x;
   const int b = xcd_bucket(blockIdx.x, a.numBuckets);
@@ -31,7 +31,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void pc
 
   for (int t0 = 0; t0 < n; t0 += kWave) {
     const int nt = min(kWave, n - t0);
-    with_targets_per_lane(nt, [&](auto kt) {
+    with_targets_per_lane<2>(nt, [&](auto kt) {
       constexpr int K = decltype(kt)::value;
       const Lanes l = lanes_for<K>(lane, nt);
       Target t[K];
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void pc
       Acc64 acc[K];
 #pragma unroll
       for (int j = 0; j < K; ++j) acc[j] = {0.0, 0.0, 0.0, 0.0, 0.0f};
-      pc_cells<PRECISE, TILE, true, K, REC>(a, start, end, cx0, cy0, cz0, t, l, rec4, acc);
+      pc_cells<PRECISE, kPcTile, true, K, REC>(a, start, end, cx0, cy0, cz0, t, l, rec4, acc);
       reduce_store<K>(rec4, l, acc, a.vars + bstart + t0);
     });
   }
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(64) void pp_kernel(ChangaGravityLaunch a) {
 
   for (int t0 = 0; t0 < n; t0 += kWave) {
     const int nt = min(kWave, n - t0);
-    with_targets_per_lane(nt, [&](auto kt) {
+    with_targets_per_lane<3, false>(nt, [&](auto kt) {
       constexpr int K = decltype(kt)::value;
       const Lanes l = lanes_for<K>(lane, nt);
       Target t[K];

@@ -126,13 +126,23 @@ __device__ __forceinline__ void pp_interact(float rx, float ry, float rz, float 
 }
 
 // Hexadecapole cell at r = tgt - cm from a staged forward record (F_ enum).
-// With the harmonic polynomials of r (not of the unit vector: the powers of
-// 1/|r| are applied at the end), V_n = Q_n . r^(n-1) (the gradients of the
-// harmonic polynomials Q_n . r^n, z eliminated by tracelessness),
-// P_n = V_n . r, d = 1/|r|, and
-//   phi -= d (m + d^4 (P2/2 + d^2 (P3/3 + d^2 P4/4)))
-//   a   += d^5 (V2 + d^2 (V3 + d^2 V4)) - d^3 S r,
-//   S = m + d^4 (5/2 P2 + d^2 (7/3 P3 + d^2 9/4 P4)).
+// With d = 1/|r|, R = d^2 r and V_n = Q_n . r^(n-1) (the contraction with the
+// harmonic polynomials of r, z eliminated by tracelessness), the polynomials
+// of rank n - 1 are formed from r and R, so that they carry d^(2(n-2)) and
+// the three ranks accumulate into one vector
+//   W = V2 + d^2 V3 + d^4 V4
+// with no separate scaling of each rank. Its partial sums give the scalars:
+// p2 = V2 . r, p23 = (V2 + d^2 V3) . r, w = W . r, and, with P_n = V_n . r,
+//   pin = m + d^4 (P2/2 + d^2 P3/3 + d^4 P4/4) = m + d^4/4 (w + (2 p2 + p23)/3),
+//   phi -= d pin,   a += d^5 W - d^3 (pin + 2 d^4 w) r
+// (the weight of P_n in a's radial term is (2n+1)/n = 1/n + 2). 111 VALU
+// instructions with the accumulation (119 with V2, V3, V4 and their powers
+// of d kept apart); in a loop of nothing else, three targets per lane, four
+// wavefronts per SIMD, 335 cycles per wavefront evaluation (347). The FP32
+// matrix instruction does not help: v_mfma_f32_4x4x1 (16 cells x 4 targets,
+// the four rows W and one scalar) shares the FMA pipe with the VALU (a
+// mixed loop takes the sum of both times, 15 x 8.2 cycles for what 57 FMAs
+// take about as long for), and measured 391 cycles.
 // The record's float4 k is rec[k * STRIDE] (STRIDE 1: records stored whole;
 // STRIDE = tile width: component planes), read by load_rec.
 // The staged record of one cell, read once per cell and evaluated for every
@@ -169,61 +179,50 @@ __device__ __forceinline__ void pc_eval(float x, float y, float z, const PcRec& 
               qxyz = c5.x, q3a = c5.y, q3b = c5.z;
   const float qxxxx = c5.w, qxyyy = c6.x, qxxxy = c6.y, qyyyy = c6.z, qxxxz = c6.w, qyyyz = c7.x,
               qxxyy = c7.y, qxxyz = c7.z, qxyyz = c7.w, q4a = c0.w, q4b = c1.x, q4c = c1.y;
-  const float x2 = x * x, y2 = y * y, z2 = z * z;
-  // rank-2 harmonic polynomials
-  const float fxx = x2 - z2, fyy = y2 - z2;
+  const float d2 = dir * dir;
+  const float X = x * d2, Y = y * d2, Z = z * d2;
+  // V2
+  float vx = qxx * x + qxy * y + qxz * z;
+  float vy = qxy * x + qyy * y + qyz * z;
+  float vz = qxz * x + qyz * y + qzz * z;
+  const float p2 = vx * x + vy * y + vz * z;
+  // rank-2 harmonic polynomials times d^2; V2 + d^2 V3
+  const float xX = x * X, yY = y * Y, zZ = z * Z;
+  const float fxx = xX - zZ, fyy = yY - zZ;
   const float x_2 = x + x, y_2 = y + y;
-  const float fxy = x_2 * y, fxz = x_2 * z, fyz = y_2 * z;
-  // rank-3 harmonic polynomials
-  const float z3 = 3.0f * z2;
-  const float fxxx = x * (x2 - z3), fyyy = y * (y2 - z3);
-  const float fxyy = (3.0f * x) * fyy, fxxy = (3.0f * y) * fxx;
-  const float fxxz = z * (3.0f * x2 - z2), fyyz = z * (3.0f * y2 - z2);
-  const float fxyz = (3.0f * z) * fxy;
-  // V2 = Q2 . r
-  const float v2x = qxx * x + qxy * y + qxz * z;
-  const float v2y = qxy * x + qyy * y + qyz * z;
-  const float v2z = qxz * x + qyz * y + qzz * z;
-  // V3 = Q3 . r r
-  const float v3x = qxxx * fxx + qxyy * fyy + qxxy * fxy + qxxz * fxz + qxyz * fyz;
-  const float v3y = qxyy * fxy + qxxy * fxx + qyyy * fyy + qyyz * fyz + qxyz * fxz;
-  const float v3z = qxxz * fxx + qyyz * fyy + qxyz * fxy + q3a * fxz + q3b * fyz;
-  // V4 = Q4 . r r r
-  const float v4x = qxxxx * fxxx + qxxyy * fxyy + qxxxy * fxxy + qxyyy * fyyy + qxxxz * fxxz +
-                    qxyyz * fyyz + qxxyz * fxyz;
-  const float v4y = qyyyy * fyyy + qxxyy * fxxy + qxxxy * fxxx + qxyyy * fxyy + qxyyz * fxyz +
-                    qxxyz * fxxz + qyyyz * fyyz;
-  const float v4z = qxxxz * fxxx + qxyyz * fxyy + qxxyz * fxxy + qyyyz * fyyy + q4a * fxxz +
-                    q4b * fyyz + q4c * fxyz;
-  const float p2 = v2x * x + v2y * y + v2z * z;
-  const float p3 = v3x * x + v3y * y + v3z * z;
-  const float p4 = v4x * x + v4y * y + v4z * z;
-  const float d2 = dir * dir, d4 = d2 * d2;
-  const float pin = m + d4 * (0.5f * p2 + d2 * ((1.0f / 3.0f) * p3 + (0.25f * d2) * p4));
-  const float S = m + d4 * (2.5f * p2 + d2 * ((7.0f / 3.0f) * p3 + (2.25f * d2) * p4));
-  const float d3 = d2 * dir, d5 = d3 * d2, d3S = d3 * S;
+  const float fxy = x_2 * Y, fxz = x_2 * Z, fyz = y_2 * Z;
+  vx += qxxx * fxx + qxyy * fyy + qxxy * fxy + qxxz * fxz + qxyz * fyz;
+  vy += qxyy * fxy + qxxy * fxx + qyyy * fyy + qyyz * fyz + qxyz * fxz;
+  vz += qxxz * fxx + qyyz * fyy + qxyz * fxy + q3a * fxz + q3b * fyz;
+  const float p23 = vx * x + vy * y + vz * z;
+  // rank-3 harmonic polynomials times d^4; W = V2 + d^2 (V3 + d^2 V4)
+  const float fxxx = X * __builtin_fmaf(-3.0f, zZ, xX), fyyy = Y * __builtin_fmaf(-3.0f, zZ, yY);
+  const float fxyy = (3.0f * X) * fyy, fxxy = (3.0f * Y) * fxx;
+  const float fxxz = Z * __builtin_fmaf(3.0f, xX, -zZ), fyyz = Z * __builtin_fmaf(3.0f, yY, -zZ);
+  const float fxyz = (3.0f * Z) * fxy;
+  vx += qxxxx * fxxx + qxxyy * fxyy + qxxxy * fxxy + qxyyy * fyyy + qxxxz * fxxz + qxyyz * fyyz +
+        qxxyz * fxyz;
+  vy += qyyyy * fyyy + qxxyy * fxxy + qxxxy * fxxx + qxyyy * fxyy + qxyyz * fxyz + qxxyz * fxxz +
+        qyyyz * fyyz;
+  vz += qxxxz * fxxx + qxyyz * fxyy + qxxyz * fxxy + qyyyz * fyyy + q4a * fxxz + q4b * fyyz +
+        q4c * fxyz;
+  const float w = vx * x + vy * y + vz * z;
+  const float d4 = d2 * d2, d3 = d2 * dir, d5 = d4 * dir;
+  const float g = __builtin_fmaf(1.0f / 3.0f, __builtin_fmaf(2.0f, p2, p23), w);
+  const float pin = __builtin_fmaf(0.25f * d4, g, m);
+  const float d3S = d3 * __builtin_fmaf(d4 + d4, w, pin);
   A.pot = __builtin_fmaf(-dir, pin, A.pot);
-  A.ax = __builtin_fmaf(d5, v2x + d2 * (v3x + d2 * v4x), A.ax);
-  A.ay = __builtin_fmaf(d5, v2y + d2 * (v3y + d2 * v4y), A.ay);
-  A.az = __builtin_fmaf(d5, v2z + d2 * (v3z + d2 * v4z), A.az);
-  A.ax = __builtin_fmaf(-d3S, x, A.ax);
-  A.ay = __builtin_fmaf(-d3S, y, A.ay);
-  A.az = __builtin_fmaf(-d3S, z, A.az);
+  A.ax = __builtin_fmaf(-d3S, x, __builtin_fmaf(d5, vx, A.ax));
+  A.ay = __builtin_fmaf(-d3S, y, __builtin_fmaf(d5, vy, A.ay));
+  A.az = __builtin_fmaf(-d3S, z, __builtin_fmaf(d5, vz, A.az));
   A.idt = max_nonneg(A.idt, (mt + m) * d3);
-}
-
-template <int STRIDE = 1>
-__device__ __forceinline__ void pc_interact(float x, float y, float z, const float4* rec,
-                                            float mt, Acc32& A) {
-  pc_eval(x, y, z, load_rec<STRIDE>(rec), mt, A);
 }
 
 // ---------------------------------------------------------------------------
 // Particle-cell kernel. Tiles of 64 cells: lane c loads cell c's 27-float
 // wire record and its ILCell, builds the staged record in registers and
-// writes it to LDS; the next tile's wire record is already in flight while
-// the current tile is evaluated. A tile without softened cells (ballot) runs
-// the hexadecapole loop with no per-cell test.
+// writes it to LDS. A tile without softened cells (ballot) runs the
+// hexadecapole loop with no per-cell test.
 // ---------------------------------------------------------------------------
 struct WireCell {
   float v[27];
@@ -258,13 +257,10 @@ __device__ __forceinline__ T load_entry(const T* p) {
   else return *p;
 }
 
-// Wire record of list entry e, for every lane (no branch: a load under a
-// divergent branch makes the compiler wait for it at the branch's end, which
-// would serialize the prefetch): the caller clamps e into the list.
-template <bool STREAM>
-__device__ __forceinline__ void load_cell_all(const ChangaGravityLaunch& a, const ILCell* cells,
-                                              int e, WireCell& w) {
-  const ILCell c = load_entry<STREAM>(cells + e);
+// Wire record of list entry c, for every lane (the caller clamps the entry
+// into the list).
+__device__ __forceinline__ void load_cell_rec(const ChangaGravityLaunch& a, const ILCell c,
+                                              WireCell& w) {
   w.idx = c.index;
   w.oid = c.offsetID;
   const float* src = reinterpret_cast<const float*>(a.moments) + (size_t)c.index * kWireStride;
@@ -520,15 +516,22 @@ __device__ __forceinline__ Lanes lanes_for(int lane, int nt) {
   return l;
 }
 
-// Targets per lane (1, 2 or 3) that keep the most target places busy,
-// nslot(K) nt / (64 K), the smaller K on ties.
+// Targets per lane (1 to LIM <= 3) that keep the most target places busy,
+// nslot(K) nt / (64 K). CELLS (the chunk runs a cell loop): the larger K on
+// ties, because every lane of a slot reads a staged cell's whole record and K
+// targets share those eight LDS reads (16 targets: 348 cycles per wavefront
+// evaluation with K = 2, 379 with K = 1), and at most two up to 16 targets
+// (K = 3 only adds places there, and the batched kernel spills for it: 128^3
+// box 2.54 ms, 2.50 with K <= 2). Particles alone (one LDS read per source):
+// the smaller K on ties (128^3 box 0.60 ms, 0.63 with the larger).
+template <int LIM = 3, bool CELLS = true>
 __device__ __forceinline__ int targets_per_lane(int nt) {
   int best = 1;
   int bnum = (kWave / nt) * nt, bden = 1;  // utilisation bnum / (64 bden)
-  for (int k = 2; k <= 3; ++k) {
+  for (int k = 2; k <= (CELLS && nt <= 16 ? 2 : LIM); ++k) {
     const int ng = (nt + k - 1) / k;
     const int num = (kWave / ng) * nt;
-    if (num * bden > bnum * k) {
+    if (num * bden + (CELLS ? 1 : 0) > bnum * k) {
       best = k;
       bnum = num;
       bden = k;
@@ -543,19 +546,17 @@ struct KTag {
 };
 
 // Calls body(KTag<K>()) with K = targets_per_lane(nt) (nt uniform across the
-// wavefront, so one of the three instantiations runs).
-template <typename Body>
+// wavefront, so one of the instantiations runs).
+template <int LIM = 3, bool CELLS = true, typename Body>
 __device__ __forceinline__ void with_targets_per_lane(int nt, Body&& body) {
-  switch (targets_per_lane(nt)) {
-    case 1:
-      body(KTag<1>());
-      break;
-    case 2:
-      body(KTag<2>());
-      break;
-    default:
-      body(KTag<3>());
-      break;
+  static_assert(LIM == 2 || LIM == 3, "targets per lane");
+  const int k = targets_per_lane<LIM, CELLS>(nt);
+  if (k == 1) {
+    body(KTag<1>());
+  } else if (LIM == 2 || k == 2) {
+    body(KTag<2>());
+  } else {
+    if constexpr (LIM == 3) body(KTag<3>());
   }
 }
 
@@ -677,12 +678,22 @@ __device__ __forceinline__ void reduce_store(void* lds, const Lanes& l, const Ac
 // planes: float4 k of cell c at rec4[k * (TILE + 1) + c], so lanes reading or
 // writing different cells touch consecutive 16-byte words (no bank
 // conflicts however many distinct cells a read instruction touches: one per
-// lane when a bucket has a single target). The next tile's data is in flight
-// while this one is evaluated. REC false: lane c fetches cell c's wire
-// record and stages it; REC true: the tile's 128-byte cell records
+// lane when a bucket has a single target). REC false: lane c fetches cell
+// c's wire record and stages it; REC true: the tile's 128-byte cell records
 // (a.cellRecords) are fetched as whole lines, eight lanes per record
 // (load_rec_tile, stage_rec_tile). A tile without softened cells (ballot)
 // runs the hexadecapole loop with no per-cell test.
+//
+// A wavefront waits for its tile's records here, and the SIMD's other three
+// wavefronts run meanwhile: holding the next tile's records in registers
+// during the evaluation (27 or 32 of them) hides that wait within a
+// wavefront but costs the fourth wavefront per SIMD or spills for it, and
+// the FP32 VALU issues the same evaluation 9% faster with four wavefronts
+// than with three (two wavefronts' FP32 instructions issue together).
+// Measured, batched graph with the tile in registers (three wavefronts;
+// one target per lane on records: four, spilling) -> without: 2^22 halos
+// 10.05 -> 9.13 ms, 128^3 box 2.65 -> 2.50, 256^3 box with a 10% rung
+// 8.71 -> 7.69; with the tile in registers at four, halos 10.8, box 2.67.
 template <bool PRECISE, int TILE, bool STREAM = true, int K = 1, bool REC = false>
 __device__ __forceinline__ void pc_cells(const ChangaGravityLaunch& a, int start, int end,
                                          double cx0, double cy0, double cz0,
@@ -701,34 +712,21 @@ __device__ __forceinline__ void pc_cells(const ChangaGravityLaunch& a, int start
   // list entry of this lane in the tile at base (clamped into the list)
   auto entry_at = [&](int base) { return min(base + min(l.lane, tc - 1), end - 1); };
   // (end - 1 >= start: the loop below runs only for a non-empty list)
-  // REC false: the next tile's wire records. REC true: the next tile's
-  // record lines, its offsetIDs, and the entries of the tile after it (read
-  // a tile ahead, so that the index shuffle of a fetch never waits on them).
   WireCell w;
   RecTile<TILE> rt;
+  // the list entries are read a tile ahead, so that a tile's fetch does not
+  // wait for its indices
   ILCell enext;
-  int oid_next = 0;
   const float4* recs = static_cast<const float4*>(a.cellRecords);
-  // every fetch is unconditional (past the list's end it fetches the last
-  // cell again): a load under any branch makes the compiler wait for it where
-  // the branch joins, which would put the fetch's latency before the
-  // evaluation it is meant to overlap
-  auto fetch = [&](int base) {
-    if constexpr (REC) {
-      load_rec_tile<TILE>(recs, enext.index, max(1, min(tc, end - base)), l.lane, rt);
-      oid_next = enext.offsetID;
-      enext = load_entry<STREAM>(cells + entry_at(base + tc));
-    } else {
-      load_cell_all<STREAM>(a, cells, entry_at(base), w);
-    }
-  };
   if (start >= end) return;
-  if constexpr (REC) enext = load_entry<STREAM>(cells + entry_at(start));
-  fetch(start);
+  enext = load_entry<STREAM>(cells + entry_at(start));
   for (int base = start; base < end; base += tc) {
     const int nc = min(tc, end - base);
     const bool mine = l.lane < nc;
-    const int oid = REC ? oid_next : w.oid;
+    const int oid = enext.offsetID;
+    if constexpr (REC) load_rec_tile<TILE>(recs, enext.index, nc, l.lane, rt);
+    else load_cell_rec(a, enext, w);
+    enext = load_entry<STREAM>(cells + entry_at(base + tc));
     const bool soft_tile = __ballot(mine && (oid & CHANGA_ILCELL_SOFTENED)) != 0ull;
     const bool shifted = tile_shifted(mine, oid);
     if constexpr (REC) {
@@ -737,8 +735,6 @@ __device__ __forceinline__ void pc_cells(const ChangaGravityLaunch& a, int start
       if (mine) stage_cell_fwd<PRECISE, PS>(a, w, L, shifted, cx0, cy0, cz0, rec4 + l.lane);
       __syncthreads();
     }
-    // issued after the barrier, whose fence would otherwise wait for them
-    fetch(base + tc);
     if (l.live) {
       Acc32 A[K];
 #pragma unroll
