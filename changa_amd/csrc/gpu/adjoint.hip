@@ -69,18 +69,18 @@ __device__ __forceinline__ D2 drsq(D2 a) {
 
 // (da/dr) w for the hexadecapole acceleration of a staged record (the
 // formula of pc_eval, evaluated on dual numbers with tangent w).
-__device__ __forceinline__ void pc_tidal(const float4* rec, float rx, float ry, float rz, float wx,
+__device__ __forceinline__ void pc_tidal(const PcRec& R, float rx, float ry, float rz, float wx,
                                          float wy, float wz, float& tx, float& ty, float& tz) {
   const D2 X = {rx, wx}, Y = {ry, wy}, Z = {rz, wz};
   const D2 dir = drsq(X * X + Y * Y + Z * Z);
-  const float4 c0 = rec[0], c1 = rec[1], c2 = rec[2], c3 = rec[3];
-  const float4 c4 = rec[4], c5 = rec[5], c6 = rec[6], c7 = rec[7];
-  const float m = c0.w;
-  const float qxx = c1.x, qxy = c1.y, qxz = c1.z, qyy = c1.w, qyz = c2.x, qzz = c2.y;
-  const float qxxx = c2.z, qxyy = c2.w, qxxy = c3.x, qyyy = c3.y, qxxz = c3.z, qyyz = c3.w,
-              qxyz = c4.x, q3a = c4.y, q3b = c4.z;
-  const float qxxxx = c4.w, qxyyy = c5.x, qxxxy = c5.y, qyyyy = c5.z, qxxxz = c5.w, qyyyz = c6.x,
-              qxxyy = c6.y, qxxyz = c6.z, qxyyz = c6.w, q4a = c7.x, q4b = c7.y, q4c = c7.z;
+  const float4 c0 = R.c0, c1 = R.c1, c2 = R.c2, c3 = R.c3, c4 = R.c4, c5 = R.c5, c6 = R.c6,
+               c7 = R.c7;
+  const float m = c1.z;
+  const float qxx = c2.x, qxy = c2.y, qxz = c2.z, qyy = c2.w, qyz = c3.x, qzz = c3.y;
+  const float qxxx = c3.z, qxyy = c3.w, qxxy = c4.x, qyyy = c4.y, qxxz = c4.z, qyyz = c4.w,
+              qxyz = c5.x, q3a = c5.y, q3b = c5.z;
+  const float qxxxx = c5.w, qxyyy = c6.x, qxxxy = c6.y, qyyyy = c6.z, qxxxz = c6.w, qyyyz = c7.x,
+              qxxyy = c7.y, qxxyz = c7.z, qxyyz = c7.w, q4a = c0.w, q4b = c1.x, q4c = c1.y;
   const D2 x = X * dir, y = Y * dir, z = Z * dir;
   const D2 x2 = x * x, y2 = y * y, z2 = z * z;
   const D2 fxx = x2 - z2, fyy = y2 - z2;
@@ -332,18 +332,71 @@ __global__ void adj_item_heads_kernel(const int* item, const int* n_owners_dev, 
   if (c < n && item[c + 1] > item[c]) owner[item[c]] = c;
 }
 
+// Sums of up to 64 values over the wavefront, value k's total to lane k: each
+// step adds the lanes' halves of the values it keeps, so the exchanges halve
+// from step to step (20, 10, 5, 3, 2, 1 for 39 values) where a butterfly per
+// value takes six each. The additions pair lanes 32, 16, 8, 4, 2, 1 apart in
+// this order, as wave_sum does: the totals are its bits.
+template <int M>
+__device__ __forceinline__ void sum_step(float* v, int lane, int n) {
+#pragma unroll
+  for (int j = 0; 2 * j < n; ++j) {
+    const float a = v[2 * j], b = 2 * j + 1 < n ? v[2 * j + 1] : 0.0f;
+    if constexpr (M >= 16) {
+      // a keeps its low lanes and takes b's low ones into its high lanes, b the rest
+      const auto r = M == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a),
+                                                                __float_as_uint(b), false, false)
+                             : __builtin_amdgcn_permlane16_swap(__float_as_uint(a),
+                                                                __float_as_uint(b), false, false);
+      v[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+      const bool odd = lane & M;
+      const float keep = odd ? b : a, send = odd ? a : b;
+      v[j] = keep + __shfl_xor(send, M, kWave);
+    }
+  }
+}
+
+template <int N>
+__device__ __forceinline__ float wave_sums(float (&v)[N], int lane) {
+  static_assert(N <= kWave, "one total per lane");
+  sum_step<32>(v, lane, N);
+  sum_step<16>(v, lane, (N + 1) / 2);
+  sum_step<8>(v, lane, (N + 3) / 4);
+  sum_step<4>(v, lane, (N + 7) / 8);
+  sum_step<2>(v, lane, (N + 15) / 16);
+  sum_step<1>(v, lane, (N + 31) / 32);
+  // lane l holds the value whose index is l's bits reversed
+  return __shfl(v[0], (int)(__brev((unsigned)lane) >> 26), kWave);
+}
+
 // ---------------------------------------------------------------------------
 // (2) cell sources: one wavefront per work item (up to kUsersPerItem users of
-// one cell); lanes walk the users' targets.
+// one cell); lanes walk the users' targets, 64 at a time. The targets of the
+// next 64 are looked up and loaded while these are evaluated. Looking up:
+// the users that begin within the window mark their first place, and a
+// lane's user is the last one begun: one ballot and a bit count, where a
+// binary search over the users took nine dependent LDS reads per target.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void adj_cells_kernel(AdjArgs a) {
-  __shared__ int u_end[kUsersPerItem];
-  __shared__ int u_start[kUsersPerItem];
+struct CellTarget {
+  double x, y, z;
+  float w0, w1, w2;
+  int i, oid;
+};
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void adj_cells_kernel(
+    AdjArgs a) {
+  __shared__ int u_from[kUsersPerItem];   // place of the user's first target among the item's
+  __shared__ int u_shift[kUsersPerItem];  // its index in the target arrays less that place
   __shared__ int u_oid[kUsersPerItem];
+  __shared__ unsigned mark[kWave];
   const int lane = threadIdx.x;
   const int n_items = a.tr.item[a.nNodes];
   const float* wire = reinterpret_cast<const float*>(a.pc.moments);
   const double L = a.pc.fperiod;
+  const unsigned long long below = (1ull << lane) - 1ull, upto = below | (1ull << lane);
+  unsigned window = 0;
+  mark[lane] = 0;
   for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
     const int c = a.tr.item_cell[it];
     const int u0 = a.tr.start[c] + (it - a.tr.item[c]) * kUsersPerItem;
@@ -351,71 +404,93 @@ __global__ __launch_bounds__(64) void adj_cells_kernel(AdjArgs a) {
     const double cx = a.pc.cm64[3 * (size_t)c], cy = a.pc.cm64[3 * (size_t)c + 1],
                  cz = a.pc.cm64[3 * (size_t)c + 2];
     const float cmass = wire[(size_t)c * 27 + 2], csoft = wire[(size_t)c * 27 + 1];
-    // users -> target ranges, prefix of their sizes
-    int base = 0;
+    // users with targets, in order -> places of their targets
+    int total = 0, users = 0;
     for (int k0 = 0; k0 < nu; k0 += kWave) {
       const int k = k0 + lane;
-      int sz = 0;
+      int sz = 0, st = 0, oid = 0;
       if (k < nu) {
         const unsigned u = a.tr.value[u0 + k];
         const int bk = (int)(u >> kBucketShift);
         sz = a.pc.sizes[bk];
-        u_start[k] = a.pc.starts[bk];
-        u_oid[k] = (int)((u & ((1u << kBucketShift) - 1u)) << 22);
+        st = a.pc.starts[bk];
+        oid = (int)((u & ((1u << kBucketShift) - 1u)) << 22);
       }
       const int incl = wave_incl_scan(sz, lane);
-      if (k < nu) u_end[k] = base + incl;
-      base += __shfl(incl, kWave - 1, kWave);
+      const unsigned long long some = __ballot(sz > 0);
+      if (sz > 0) {
+        const int at = users + __popcll(some & below), from = total + incl - sz;
+        u_from[at] = from;
+        u_shift[at] = st - from;
+        u_oid[at] = oid;
+      }
+      users += __popcll(some);
+      total += __shfl(incl, kWave - 1, kWave);
     }
     __syncthreads();
-    const int total = base;
-    float D[36];
+    float D[39];  // 36 tensor components, then the softened cells' sum
 #pragma unroll
-    for (int k = 0; k < 36; ++k) D[k] = 0.0f;
-    float vs0 = 0.f, vs1 = 0.f, vs2 = 0.f;
+    for (int k = 0; k < 39; ++k) D[k] = 0.0f;
+    int begun = 0;  // users begun before the next window
+    // the targets at places [q0, q0 + 64) (past the end: the last one again)
+    auto fetch = [&](int q0, CellTarget& t) {
+      ++window;
+      if (begun + lane < users) {
+        const int f = u_from[begun + lane] - q0;
+        if (f < kWave) mark[f] = window;
+      }
+      __syncthreads();
+      const unsigned long long m = __ballot(mark[lane] == window);
+      const int k = begun + __popcll(m & upto) - 1;
+      begun += __popcll(m);
+      t.oid = u_oid[k];
+      t.i = u_shift[k] + min(q0 + lane, total - 1);
+      const double* p = a.pc.tpos64 + 3 * (size_t)t.i;
+      t.x = p[0];
+      t.y = p[1];
+      t.z = p[2];
+      const float* w = a.w + 3 * (size_t)t.i;
+      t.w0 = w[0];
+      t.w1 = w[1];
+      t.w2 = w[2];
+    };
+    CellTarget nx;
+    if (total > 0) fetch(0, nx);
     for (int q0 = 0; q0 < total; q0 += kWave) {
-      const int q = q0 + lane;
-      if (q < total) {
-        const int k = find_run(u_end, nu, q);
-        const int oid = u_oid[k];
-        const int i = u_start[k] + q - (k ? u_end[k - 1] : 0);
-        const float rx = (float)(a.pc.tpos64[3 * (size_t)i] - (cx + off_x(oid) * L));
-        const float ry = (float)(a.pc.tpos64[3 * (size_t)i + 1] - (cy + off_y(oid) * L));
-        const float rz = (float)(a.pc.tpos64[3 * (size_t)i + 2] - (cz + off_z(oid) * L));
-        const float wx = a.w[3 * (size_t)i], wy = a.w[3 * (size_t)i + 1],
-                    wz = a.w[3 * (size_t)i + 2];
-        const float r2 = rx * rx + ry * ry + rz * rz;
-        if (r2 != 0.0f) {
-          if (oid & CHANGA_ILCELL_SOFTENED) {
-            // monopole pseudo-particle at the cm: d = -r
-            float bb, cc;
-            spline_bc(r2, a.pc.targets[i].soft + csoft, bb, cc);
-            const float dw = -(rx * wx + ry * wy + rz * wz);
-            D[0] += bb * dw;
-            vs0 -= cmass * (bb * wx + cc * rx * dw);
-            vs1 -= cmass * (bb * wy + cc * ry * dw);
-            vs2 -= cmass * (bb * wz + cc * rz * dw);
-          } else {
-            const float ir = rsq(r2);
-            accumulate_d(rx, ry, rz, ir, ir * ir, wx, wy, wz, D);
-          }
+      const bool mine = q0 + lane < total;
+      const int oid = nx.oid, i = nx.i;
+      const float wx = nx.w0, wy = nx.w1, wz = nx.w2;
+      float rx, ry, rz;
+      if (tile_shifted(mine, oid)) {
+        rx = (float)(nx.x - (cx + off_x(oid) * L));
+        ry = (float)(nx.y - (cy + off_y(oid) * L));
+        rz = (float)(nx.z - (cz + off_z(oid) * L));
+      } else {
+        rx = (float)(nx.x - cx);
+        ry = (float)(nx.y - cy);
+        rz = (float)(nx.z - cz);
+      }
+      fetch(min(q0 + kWave, total - 1), nx);
+      const float r2 = rx * rx + ry * ry + rz * rz;
+      if (mine && r2 != 0.0f) {
+        if (oid & CHANGA_ILCELL_SOFTENED) {
+          // monopole pseudo-particle at the cm: d = -r
+          float bb, cc;
+          spline_bc(r2, a.pc.targets[i].soft + csoft, bb, cc);
+          const float dw = -(rx * wx + ry * wy + rz * wz);
+          D[0] += bb * dw;
+          D[36] -= cmass * (bb * wx + cc * rx * dw);
+          D[37] -= cmass * (bb * wy + cc * ry * dw);
+          D[38] -= cmass * (bb * wz + cc * rz * dw);
+        } else {
+          const float ir = rsq(r2);
+          accumulate_d(rx, ry, rz, ir, ir * ir, wx, wy, wz, D);
         }
       }
     }
     // reduce across the wavefront; lane k adds component k
+    const float mine = wave_sums(D, lane);
     double* nd = a.node + (size_t)c * kAdjStride;
-    float mine = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 36; ++k) {
-      const float s = wave_sum(D[k]);
-      if (lane == k) mine = s;
-    }
-    {
-      const float s0 = wave_sum(vs0), s1 = wave_sum(vs1), s2 = wave_sum(vs2);
-      if (lane == 36) mine = s0;
-      if (lane == 37) mine = s1;
-      if (lane == 38) mine = s2;
-    }
     if (lane < 39 && mine != 0.0f) atomicAdd(nd + lane, (double)mine);
     __syncthreads();
   }
@@ -568,19 +643,27 @@ __global__ __launch_bounds__(64) void adj_pp_sources_kernel(AdjArgs a) {
 // ---------------------------------------------------------------------------
 template <int KIND>
 struct TargetsLds {
-  static constexpr size_t pc = (size_t)kAdjPcTile * kPcRec * sizeof(float);
+  static constexpr size_t pc = (size_t)(kAdjPcTile + 1) * kFwdRec * sizeof(float);
   static constexpr size_t pp = sizeof(PpLds<kPpTile>);
   static constexpr size_t bytes = pc > pp ? pc : pp;
   static constexpr size_t f4 = (bytes + 15) / 16;
 };
 
-template <int KIND>
-__global__ __launch_bounds__(64) void adj_targets_kernel(AdjArgs a) {
+// REC: cells from the 128-byte cell records (a.pc.cellRecords), else from the
+// wire moments (the same staged bits). Four wavefronts per SIMD and the
+// component planes of the forward loops, for their reasons (gravity_body.h:
+// pc_cells).
+template <int KIND, bool REC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void adj_targets_kernel(
+    AdjArgs a) {
   __shared__ float4 lds[TargetsLds<KIND>::f4];
-  __shared__ float4 tp4[kWave];  // target x, y, z (bucket-centred), softening
-  __shared__ float4 tw4[kWave];  // w
+  // the chunk's targets, for the source side of per-particle lists: x, y, z
+  // (bucket-centred), softening; w
+  __shared__ float4 tp4[KIND == 0 ? kWave : 1];
+  __shared__ float4 tw4[KIND == 0 ? kWave : 1];
   float4* rec4 = lds;
   PpLds<kPpTile>& ps = *reinterpret_cast<PpLds<kPpTile>*>(lds);
+  constexpr int PS = kAdjPcTile + 1;
 
   const int lane = threadIdx.x;
   const int b = xcd_bucket(blockIdx.x, a.pc.numBuckets);
@@ -588,54 +671,69 @@ __global__ __launch_bounds__(64) void adj_targets_kernel(AdjArgs a) {
   const int pps = a.pp.marks[b], ppe = a.pp.marks[b + 1];
   const int bstart = a.pc.starts[b], n = a.pc.sizes[b];
   const float L = a.pc.fperiod;
+  const Period period = {L, L, L};
   double cx0, cy0, cz0;
   bucket_centre<true>(a.pc.tpos64, bstart, n, cx0, cy0, cz0);
   const ILCell* cells = static_cast<const ILCell*>(a.pc.list);
+  const float4* recs = static_cast<const float4*>(a.pc.cellRecords);
 
   for (int t0 = 0; t0 < n; t0 += kWave) {
     const int nt = min(kWave, n - t0);
     const Lanes l = lanes_for(lane, nt);
-    if (lane < nt) {
-      const int tp = bstart + t0 + lane;
-      tp4[lane] = make_float4((float)(a.pc.tpos64[3 * (size_t)tp] - cx0),
-                              (float)(a.pc.tpos64[3 * (size_t)tp + 1] - cy0),
-                              (float)(a.pc.tpos64[3 * (size_t)tp + 2] - cz0),
-                              a.pc.targets[tp].soft);
-      tw4[lane] = make_float4(a.w[3 * (size_t)tp], a.w[3 * (size_t)tp + 1],
-                              a.w[3 * (size_t)tp + 2], 0.0f);
+    auto target = [&](int j, float4& pos, float4& w) {
+      const int tp = bstart + t0 + j;
+      pos = make_float4((float)(a.pc.tpos64[3 * (size_t)tp] - cx0),
+                        (float)(a.pc.tpos64[3 * (size_t)tp + 1] - cy0),
+                        (float)(a.pc.tpos64[3 * (size_t)tp + 2] - cz0), a.pc.targets[tp].soft);
+      w = make_float4(a.w[3 * (size_t)tp], a.w[3 * (size_t)tp + 1], a.w[3 * (size_t)tp + 2], 0.0f);
+    };
+    if constexpr (KIND == 0) {
+      if (lane < nt) target(lane, tp4[lane], tw4[lane]);
+      __syncthreads();
     }
-    __syncthreads();
-    const int j = l.live ? l.lane - l.slot * l.nt : 0;
-    const float4 me = tp4[j], mw = tw4[j];
+    float4 me, mw;
+    target(l.live ? l.lane - l.slot * l.nt : 0, me, mw);
     double ax = 0.0, ay = 0.0, az = 0.0;
 
     // ---- cells, target side
-    WireCell wc;
-    wc.oid = 0;
-    load_cell<true>(a.pc, cells, pcs + lane, pce, wc);
+    ILCell enext = {0, 0};
+    if (pcs < pce) enext = load_entry<true>(cells + min(pcs + lane, pce - 1));
     for (int base = pcs; base < pce; base += kAdjPcTile) {
       const int nc = min(kAdjPcTile, pce - base);
-      if (lane < nc) stage_cell<true>(a.pc, wc, L, cx0, cy0, cz0, rec4 + lane * (kPcRec / 4));
-      __syncthreads();
-      load_cell<true>(a.pc, cells, base + kAdjPcTile + lane, pce, wc);
+      const int oid = enext.offsetID;
+      const bool shifted = tile_shifted(lane < nc, oid);
+      if constexpr (REC) {
+        RecTile<kAdjPcTile> rt;
+        load_rec_tile<kAdjPcTile>(recs, enext.index, nc, lane, rt);
+        enext = load_entry<true>(cells + min(base + kAdjPcTile + lane, pce - 1));
+        stage_rec_tile<true, kAdjPcTile, PS>(rt, nc, lane, oid, period, shifted, cx0, cy0, cz0,
+                                             rec4);
+      } else {
+        WireCell wc;
+        load_cell_rec(a.pc, enext, wc);
+        enext = load_entry<true>(cells + min(base + kAdjPcTile + lane, pce - 1));
+        if (lane < nc)
+          stage_cell_fwd<true, PS>(a.pc, wc, period, shifted, cx0, cy0, cz0, rec4 + lane);
+        __syncthreads();
+      }
       if (l.live) {
         float sx = 0.f, sy = 0.f, sz = 0.f;
         for (int c = l.slot; c < nc; c += l.nslot) {
-          const float4* r4 = rec4 + c * (kPcRec / 4);
-          const float4 h = r4[0];
-          const float rx = me.x - h.x, ry = me.y - h.y, rz = me.z - h.z;
+          const PcRec R = load_rec<PS>(rec4 + c);
+          const float rx = me.x - R.c0.x, ry = me.y - R.c0.y, rz = me.z - R.c0.z;
           const float r2 = rx * rx + ry * ry + rz * rz;
           if (r2 == 0.0f) continue;
           float tx, ty, tz;
-          if (h.w < 0.0f) {  // softened: spline monopole at the cm (d = -r)
+          if (R.c1.w >= 0.0f) {  // softened: spline monopole at the cm (d = -r)
+            const float m = -R.c1.z;
             float bb, cc;
-            spline_bc(r2, me.w + r4[1].x, bb, cc);
+            spline_bc(r2, me.w + R.c1.w, bb, cc);
             const float dw = -(rx * mw.x + ry * mw.y + rz * mw.z);
-            tx = h.w * (bb * mw.x + cc * rx * dw);
-            ty = h.w * (bb * mw.y + cc * ry * dw);
-            tz = h.w * (bb * mw.z + cc * rz * dw);
+            tx = m * (bb * mw.x + cc * rx * dw);
+            ty = m * (bb * mw.y + cc * ry * dw);
+            tz = m * (bb * mw.z + cc * rz * dw);
           } else {
-            pc_tidal(r4, rx, ry, rz, mw.x, mw.y, mw.z, tx, ty, tz);
+            pc_tidal(R, rx, ry, rz, mw.x, mw.y, mw.z, tx, ty, tz);
           }
           sx += tx;
           sy += ty;
@@ -1624,10 +1722,14 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
     CGPU_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     hipLaunchKernelGGL(adj_cells_kernel, dim3(ncu * 16), dim3(kWave), 0, s, args);
     CGPU_CHECK(hipGetLastError());
-    if (pp.listKind == 1)
-      hipLaunchKernelGGL(adj_targets_kernel<1>, dim3(nb), dim3(kWave), 0, s, args);
-    else
-      hipLaunchKernelGGL(adj_targets_kernel<0>, dim3(nb), dim3(kWave), 0, s, args);
+    // (records that are not line-aligned are left aside: the wire moments
+    // hold the same values)
+    const bool rec = args.pc.cellRecords &&
+                     reinterpret_cast<uintptr_t>(args.pc.cellRecords) % CHANGA_CELL_RECORD_BYTES == 0;
+    const auto targets = pp.listKind == 1
+                             ? (rec ? adj_targets_kernel<1, true> : adj_targets_kernel<1, false>)
+                             : (rec ? adj_targets_kernel<0, true> : adj_targets_kernel<0, false>);
+    hipLaunchKernelGGL(targets, dim3(nb), dim3(kWave), 0, s, args);
     CGPU_CHECK(hipGetLastError());
     if (R > 0) {
       hipLaunchKernelGGL(adj_pp_sources_kernel, dim3(ncu * 16), dim3(kWave), 0, s, args);

@@ -27,30 +27,13 @@
 namespace cgpu {
 
 constexpr int kPcTile = 64;   // cells per staged tile of the plain kernel
-constexpr int kPcRec = 36;    // floats per staged cell record of the adjoint's target pass
-                              // (9 x float4, stored whole: 36 keeps records read together
-                              // 4 LDS banks apart)
 constexpr int kFwdRec = 32;   // floats per staged cell record of the forward loops
                               // (8 float4 component planes)
 constexpr int kPpTile = 256;  // source particles per staged tile
 
-// Staged cell record of the adjoint's target pass (36 floats). Moments of
-// order n are multiplied by n c_n radius^n (c_n = (2n-1)!!/n!), the replica
-// offset is applied to the centre, and the combinations the trace-free
-// contraction needs are formed once per cell. A cell whose softening
-// overlaps the bucket is stored with negative mass and its softening in
-// slot 4.
-enum {
-  R_CX = 0, R_CY, R_CZ, R_M,
-  R_Q2 = 4,    // xx xy xz yy yz, then -(xx+yy)
-  R_Q3 = 10,   // xxx xyy xxy yyy xxz yyz xyz, then -(xxx+xyy), -(xxy+yyy)
-  R_Q4 = 19,   // xxxx xyyy xxxy yyyy xxxz yyyz xxyy xxyz xyyz,
-               // then -(xxxx+xxyy), -(yyyy+xxyy), -(xxxy+xyyy)
-  R_SOFT = 4
-};
-
-// Staged cell record of the forward loops (32 floats, 8 float4): the same
-// scaled moments and trace combinations, with the centre (replica offset
+// Staged cell record (32 floats, 8 float4): moments of order n multiplied by
+// n c_n radius^n (c_n = (2n-1)!!/n!), the combinations the trace-free
+// contraction needs, formed once per cell, the centre (replica offset
 // applied, relative to the bucket centre in the precision form) in the first
 // three floats, the mass in F_M and, in F_SOFT, the cell's softening when
 // its softening overlaps the bucket (a spline monopole) or -1 for a
@@ -266,64 +249,6 @@ __device__ __forceinline__ void load_cell_rec(const ChangaGravityLaunch& a, cons
   const float* src = reinterpret_cast<const float*>(a.moments) + (size_t)c.index * kWireStride;
 #pragma unroll
   for (int k = 0; k < 27; ++k) w.v[k] = src[wire_float(k)];
-}
-
-template <bool PRECISE, bool STREAM = true>
-__device__ __forceinline__ void load_cell(const ChangaGravityLaunch& a, const ILCell* cells, int e,
-                                          int end, WireCell& w) {
-  if (e < end) {
-    const ILCell c = load_entry<STREAM>(cells + e);
-    w.idx = c.index;
-    w.oid = c.offsetID;
-    const float* src = reinterpret_cast<const float*>(a.moments) + (size_t)c.index * kWireStride;
-#pragma unroll
-    for (int k = 0; k < 27; ++k) w.v[k] = src[wire_float(k)];
-  }
-}
-
-// wire record -> staged record (in registers), then to LDS (float4 k at
-// dst[k * STRIDE])
-template <bool PRECISE, int STRIDE = 1>
-__device__ __forceinline__ void stage_cell(const ChangaGravityLaunch& a, const WireCell& w, float L,
-                                           double cx0, double cy0, double cz0, float4* dst) {
-  // wire: 0 radius, 1 soft, 2 mass, 3-5 cm, 6-10 Q2 (xx xy xz yy yz),
-  // 11-17 Q3 (xxx xyy xxy yyy xxz yyz xyz), 18-26 Q4
-  float r[kPcRec];
-  const int oid = w.oid;
-  if (PRECISE) {
-    const size_t ci = (size_t)w.idx * 3;
-    r[R_CX] = (float)(a.cm64[ci] + (double)off_x(oid) * (double)L - cx0);
-    r[R_CY] = (float)(a.cm64[ci + 1] + (double)off_y(oid) * (double)L - cy0);
-    r[R_CZ] = (float)(a.cm64[ci + 2] + (double)off_z(oid) * (double)L - cz0);
-  } else {
-    r[R_CX] = (float)off_x(oid) * L + w.v[3];
-    r[R_CY] = (float)off_y(oid) * L + w.v[4];
-    r[R_CZ] = (float)off_z(oid) * L + w.v[5];
-  }
-  const float u = w.v[0], u2 = u * u;
-  const float s2 = 3.0f * u2, s3 = 7.5f * u2 * u, s4 = 17.5f * u2 * u2;
-#pragma unroll
-  for (int k = 0; k < 5; ++k) r[R_Q2 + k] = s2 * w.v[6 + k];
-  r[R_Q2 + 5] = -(r[R_Q2 + 0] + r[R_Q2 + 3]);
-#pragma unroll
-  for (int k = 0; k < 7; ++k) r[R_Q3 + k] = s3 * w.v[11 + k];
-  r[R_Q3 + 7] = -(r[R_Q3 + 0] + r[R_Q3 + 1]);
-  r[R_Q3 + 8] = -(r[R_Q3 + 2] + r[R_Q3 + 3]);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) r[R_Q4 + k] = s4 * w.v[18 + k];
-  r[R_Q4 + 9] = -(r[R_Q4 + 0] + r[R_Q4 + 6]);
-  r[R_Q4 + 10] = -(r[R_Q4 + 3] + r[R_Q4 + 6]);
-  r[R_Q4 + 11] = -(r[R_Q4 + 2] + r[R_Q4 + 1]);
-#pragma unroll
-  for (int k = R_Q4 + 12; k < kPcRec; ++k) r[k] = 0.0f;
-  r[R_M] = w.v[2];
-  if (oid & CHANGA_ILCELL_SOFTENED) {
-    r[R_M] = -w.v[2];
-    r[R_SOFT] = w.v[1];
-  }
-#pragma unroll
-  for (int k = 0; k < kPcRec / 4; ++k)
-    dst[k * STRIDE] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
 }
 
 // Replica code of the central image (x, y, z offsets 0) in offsetID bits
