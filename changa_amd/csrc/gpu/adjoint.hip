@@ -24,7 +24,7 @@
 // differentiated).
 //
 // Passes: (1) the cell list is transposed on the GPU: a stable radix sort of
-// the entries by cell (rocPRIM) gives, for every cell, the (bucket, replica)
+// the entries by cell (transpose.h) gives, for every cell, the (bucket, replica)
 // pairs that use it in bucket order; (2) a persistent cell-major kernel
 // accumulates D for chunks of each cell's users, one wave per chunk, lanes
 // over the users' targets; (3) a bucket-major kernel adds the target-side
@@ -40,6 +40,7 @@
 #include "ewald_body.h"
 #include "gravity_body.h"
 #include "stf.h"
+#include "transpose.h"
 
 namespace cgpu {
 
@@ -243,15 +244,16 @@ __device__ __forceinline__ int find_run(const int* ends, int n, int q) {
 }
 
 // Transposed cell lists (scratch):
-//   key[E], value[E] (the entries as sorted: cell, then {bucket, replica and
-//   softened bits of offsetID} packed in 32 bits), start[nNodes + 1] (users
-//   of cell c at [start[c], start[c+1])), chunks[nNodes + 1], item[nNodes + 1]
-//   (work items per cell, exclusive prefix; item[nNodes] is their number),
-//   item_cell[items] (the cell of each item).
+//   key[E], value[E] (the entries grouped by cell: cell, then {bucket, replica
+//   and softened bits of offsetID} packed in 32 bits), start[nNodes],
+//   end[nNodes] (users of cell c at [start[c], end[c])), chunks[nNodes + 1],
+//   item[nNodes + 1] (work items per cell, exclusive prefix; item[nNodes] is
+//   their number), item_cell[items] (the cell of each item).
 struct Transpose {
   const unsigned* key;
   const unsigned* value;  // bucket << kBucketShift | offsetID >> 22
   int* start;
+  int* end;
   int* chunks;
   int* item;
   int* item_cell;  // cell of each work item
@@ -286,40 +288,35 @@ struct AdjArgs {
 // ---------------------------------------------------------------------------
 // (1) transpose
 // ---------------------------------------------------------------------------
-// value: bucket << 10 | offsetID bits 31..22 (replica and softened flag;
-// bits 21..0 carry no information for a cell entry)
-constexpr int kBucketShift = 10;
 constexpr int kMaxAdjBuckets = 1 << 22;
 
-__global__ __launch_bounds__(64) void adj_keys_kernel(ChangaGravityLaunch pc, unsigned* key,
-                                                      unsigned* value) {
-  const int b = blockIdx.x;
-  const ILCell* cells = static_cast<const ILCell*>(pc.list);
-  for (int e = pc.marks[b] + threadIdx.x; e < pc.marks[b + 1]; e += kWave) {
-    const ILCell c = cells[e];
-    key[e] = (unsigned)c.index;
-    value[e] = ((unsigned)b << kBucketShift) | ((unsigned)c.offsetID >> 22);
+// The entries of cell c are [start[c], end[c]) of the grouped list (both 0 for
+// a cell without users: the arrays are cleared before).
+constexpr int kBoundsPer = 4;  // entries per thread: one read of each key, and one of its neighbours'
+__global__ void adj_bounds_kernel(const unsigned* key, int entries, int* start, int* end) {
+  const long long k0 = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * kBoundsPer;
+  if (k0 >= entries) return;
+  const int k = (int)k0, m = min(kBoundsPer, entries - k);
+  unsigned c[kBoundsPer];
+#pragma unroll
+  for (int j = 0; j < kBoundsPer; ++j) c[j] = j < m ? key[k + j] : 0u;
+  if (k == 0 || key[k - 1] != c[0]) start[c[0]] = k;
+#pragma unroll
+  for (int j = 0; j < kBoundsPer; ++j) {
+    if (j >= m) break;
+    const bool last = k + j == entries - 1;
+    const unsigned next = last ? 0u : (j + 1 < kBoundsPer && j + 1 < m ? c[(j + 1) % kBoundsPer]
+                                                                       : key[k + j + 1]);
+    if (last || next != c[j]) {
+      end[c[j]] = k + j + 1;
+      if (!last && j + 1 < m) start[next] = k + j + 1;
+    }
   }
 }
 
-// start[c] = first sorted position whose cell is >= c
-__global__ void adj_bounds_kernel(const unsigned* key, int entries, int n_nodes, int* start) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (entries == 0) {
-    if (k <= n_nodes) start[k] = 0;
-    return;
-  }
-  if (k >= entries) return;
-  const int hi = (int)key[k];
-  const int lo = k ? (int)key[k - 1] + 1 : 0;
-  for (int c = lo; c <= hi; ++c) start[c] = k;
-  if (k == entries - 1)
-    for (int c = hi + 1; c <= n_nodes; ++c) start[c] = entries;
-}
-
-__global__ void adj_chunks_kernel(const int* start, int n_nodes, int* chunks) {
+__global__ void adj_chunks_kernel(const int* start, const int* end, int n_nodes, int* chunks) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n_nodes) chunks[c] = (start[c + 1] - start[c] + kUsersPerItem - 1) / kUsersPerItem;
+  if (c < n_nodes) chunks[c] = (end[c] - start[c] + kUsersPerItem - 1) / kUsersPerItem;
   if (c == n_nodes) chunks[c] = 0;
 }
 
@@ -400,7 +397,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ad
   for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
     const int c = a.tr.item_cell[it];
     const int u0 = a.tr.start[c] + (it - a.tr.item[c]) * kUsersPerItem;
-    const int nu = min(kUsersPerItem, a.tr.start[c + 1] - u0);
+    const int nu = min(kUsersPerItem, a.tr.end[c] - u0);
     const double cx = a.pc.cm64[3 * (size_t)c], cy = a.pc.cm64[3 * (size_t)c + 1],
                  cz = a.pc.cm64[3 * (size_t)c + 2];
     const float cmass = wire[(size_t)c * 27 + 2], csoft = wire[(size_t)c * 27 + 1];
@@ -1440,7 +1437,7 @@ static int item_owners(const int* item, const int* n_owners_dev, int n_owners, i
 
 // Scratch layout of listWork (offsets in ints, 256-byte aligned segments).
 struct WorkLayout {
-  size_t key, key_out, val, val_out, start, chunks, item, item_cell;
+  size_t sort0, sort1, counts, start, end, chunks, item, item_cell;
   size_t pkey, pkey_out, pval, pval_out, puniq, pcount, pstart, pnruns, pchunks, pitem, pitem_run;
   size_t item_cap, pitem_cap, item_heads, pitem_heads;
   size_t temp, total;
@@ -1461,11 +1458,8 @@ static hipError_t work_layout(int n_nodes, int entries, int part_entries, int n_
                               WorkLayout& L) {
   L.end_bit = bits_for(n_nodes);
   L.p_end_bit = bits_for(n_particles);
-  size_t sort_bytes = 0, scan_bytes = 0, psort_bytes = 0, rle_bytes = 0, pscan_bytes = 0;
-  hipError_t e = rocprim::radix_sort_pairs(nullptr, sort_bytes, (const unsigned*)nullptr,
-                                           (unsigned*)nullptr, (const unsigned*)nullptr,
-                                           (unsigned*)nullptr, (size_t)entries, 0, L.end_bit);
-  if (e != hipSuccess) return e;
+  size_t scan_bytes = 0, psort_bytes = 0, rle_bytes = 0, pscan_bytes = 0;
+  hipError_t e;
   e = rocprim::exclusive_scan(nullptr, scan_bytes, (const int*)nullptr, (int*)nullptr, 0,
                               (size_t)n_nodes + 1, rocprim::plus<int>());
   if (e != hipSuccess) return e;
@@ -1495,7 +1489,7 @@ static hipError_t work_layout(int n_nodes, int entries, int part_entries, int n_
                                 pitem_cap, rocprim::maximum<int>());
     if (e != hipSuccess) return e;
   }
-  size_t tb = sort_bytes;
+  size_t tb = 0;
   for (size_t x : {scan_bytes, psort_bytes, rle_bytes, pscan_bytes, own_bytes, pown_bytes})
     tb = x > tb ? x : tb;
   L.temp_bytes = tb;
@@ -1506,11 +1500,11 @@ static hipError_t work_layout(int n_nodes, int entries, int part_entries, int n_
     o = align64(o + ints);
     return at;
   };
-  L.key = take(E);
-  L.key_out = take(E);
-  L.val = take(E);
-  L.val_out = take(E);
-  L.start = take((size_t)n_nodes + 1);
+  L.sort0 = take(2 * E);
+  L.sort1 = take(2 * E);
+  L.counts = take(tr_count_ints(tr_plan(entries, (int)L.end_bit)));
+  L.start = take((size_t)n_nodes);
+  L.end = take((size_t)n_nodes);
   L.chunks = take((size_t)n_nodes + 1);
   L.item = take((size_t)n_nodes + 1);
   L.item_cap = (size_t)n_nodes + E / kUsersPerItem + 1;
@@ -1632,10 +1626,6 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
   if (int e = zero(a->grad, 4 * (size_t)a->nParticles, s)) return e;
   if (int e = zero(a->nodeWork, (size_t)kAdjStride * nn, s)) return e;
   int* iw = a->listWork;
-  unsigned* key = reinterpret_cast<unsigned*>(iw + W.key);
-  unsigned* key_out = reinterpret_cast<unsigned*>(iw + W.key_out);
-  unsigned* val = reinterpret_cast<unsigned*>(iw + W.val);
-  unsigned* val_out = reinterpret_cast<unsigned*>(iw + W.val_out);
   AdjArgs args;
   args.pc = pc;
   args.pp = pp;
@@ -1645,9 +1635,8 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
   args.node = a->nodeWork;
   args.nNodes = nn;
   args.entries = E;
-  args.tr.key = key_out;
-  args.tr.value = val_out;
   args.tr.start = iw + W.start;
+  args.tr.end = iw + W.end;
   args.tr.chunks = iw + W.chunks;
   args.tr.item = iw + W.item;
   args.tr.item_cell = iw + W.item_cell;
@@ -1658,22 +1647,25 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
   args.ptr.item = iw + W.pitem;
   args.ptr.item_run = iw + W.pitem_run;
   // (1) transpose: entries sorted by cell, stable (bucket order within a cell)
-  if (nb > 0) {
-    hipLaunchKernelGGL(adj_keys_kernel, dim3(nb), dim3(kWave), 0, s, pc, key, val);
-    CGPU_CHECK(hipGetLastError());
-  }
-  if (E > 0) {
-    size_t tb = W.temp_bytes;
-    CGPU_CHECK(rocprim::radix_sort_pairs(iw + W.temp, tb, key, key_out, val, val_out, (size_t)E,
-                                         0, W.end_bit, s));
-  }
+  args.tr.key = args.tr.value = nullptr;
+  if (E > 0)
+    if (int e = tr_sort(pc, E, (int)W.end_bit, iw + W.sort0, iw + W.sort1, iw + W.counts,
+                        &args.tr.key, &args.tr.value, s))
+      return e;
   {
-    const int n = E > nn + 1 ? E : nn + 1;
-    hipLaunchKernelGGL(adj_bounds_kernel, dim3((n + 255) / 256), dim3(256), 0, s, key_out, E, nn,
-                       args.tr.start);
+    // start and end lie one behind the other
+    const size_t bounds = W.end + (size_t)nn - W.start;
+    hipLaunchKernelGGL(fill_zero_int_kernel, dim3((unsigned)((bounds + 255) / 256)), dim3(256), 0,
+                       s, args.tr.start, bounds);
     CGPU_CHECK(hipGetLastError());
+    if (E > 0) {
+      constexpr size_t per = 256 * kBoundsPer;
+      hipLaunchKernelGGL(adj_bounds_kernel, dim3((unsigned)(((size_t)E + per - 1) / per)),
+                         dim3(256), 0, s, args.tr.key, E, args.tr.start, args.tr.end);
+      CGPU_CHECK(hipGetLastError());
+    }
     hipLaunchKernelGGL(adj_chunks_kernel, dim3((nn + 1 + 255) / 256), dim3(256), 0, s,
-                       args.tr.start, nn, args.tr.chunks);
+                       args.tr.start, args.tr.end, nn, args.tr.chunks);
     CGPU_CHECK(hipGetLastError());
     size_t tb = W.temp_bytes;
     CGPU_CHECK(rocprim::exclusive_scan(iw + W.temp, tb, args.tr.chunks, args.tr.item, 0,
