@@ -26,11 +26,120 @@
 // keeps only the lattice vectors any of them can need (compacted into LDS),
 // then every lane applies the exact per-particle test. The h-loop table is
 // staged in LDS (dynamic size; no 80-entry limit).
+//
+// Bound by FP32 VALU issue: about 80 replica terms of 165 instructions and 73
+// k-space pairs of 26 per particle. 2^21 particles take 0.68 ms (0.92 with
+// library error functions, 185 instructions a term, all 146 k-space entries,
+// divisions in the candidate search and four wavefronts per SIMD).
 #include "ewald_body.h"
 
 namespace cgpu {
 
-__global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* parts,
+// The root's moments for the FP32 replica terms: Q_n / n! with the trace
+// combinations formed, one value for the whole wavefront (scalar registers:
+// 25 vector registers fewer, so five wavefronts per SIMD instead of four).
+struct EwaldMom32 {
+  float m, xx, yy, xy, xz, yz, zz;
+  float xxx, xyy, xxy, yyy, xxz, yyz, xyz, q3a, q3b;
+  float xxxx, xyyy, xxxy, yyyy, xxxz, yyyz, xxyy, xxyz, xyyz, q4a, q4b, q4c;
+};
+
+__device__ __forceinline__ float uniform(double v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int((float)v)));
+}
+
+__device__ __forceinline__ EwaldMom32 ewald_mom32(const Mom22<double>& Q) {
+  const double h = 0.5, s = 1.0 / 6.0, f = 1.0 / 24.0;
+  EwaldMom32 o;
+  o.m = uniform(Q.m);
+  o.xx = uniform(h * Q.xx); o.yy = uniform(h * Q.yy); o.xy = uniform(h * Q.xy);
+  o.xz = uniform(h * Q.xz); o.yz = uniform(h * Q.yz); o.zz = uniform(-h * (Q.xx + Q.yy));
+  o.xxx = uniform(s * Q.xxx); o.xyy = uniform(s * Q.xyy); o.xxy = uniform(s * Q.xxy);
+  o.yyy = uniform(s * Q.yyy); o.xxz = uniform(s * Q.xxz); o.yyz = uniform(s * Q.yyz);
+  o.xyz = uniform(s * Q.xyz);
+  o.q3a = uniform(-s * (Q.xxx + Q.xyy)); o.q3b = uniform(-s * (Q.xxy + Q.yyy));
+  o.xxxx = uniform(f * Q.xxxx); o.xyyy = uniform(f * Q.xyyy); o.xxxy = uniform(f * Q.xxxy);
+  o.yyyy = uniform(f * Q.yyyy); o.xxxz = uniform(f * Q.xxxz); o.yyyz = uniform(f * Q.yyyz);
+  o.xxyy = uniform(f * Q.xxyy); o.xxyz = uniform(f * Q.xxyz); o.xyyz = uniform(f * Q.xyyz);
+  o.q4a = uniform(-f * (Q.xxxx + Q.xxyy)); o.q4b = uniform(-f * (Q.yyyy + Q.xxyy));
+  o.q4c = uniform(-f * (Q.xxxy + Q.xyyy));
+  return o;
+}
+
+// One replica term (ewald_term's sums) with V_n = Q_n . r^(n-1) / n! and
+// p_n = V_n . r:  pot = -(g0 m + g2 p2 + g3 p3 + g4 p4),
+//   a = 2 g2 V2 + 3 g3 V3 + 4 g4 V4 - (g1 m + g3 p2 + g4 p3 + g5 p4) r.
+__device__ __forceinline__ void ewald_term32(const EwaldMom32& Q, float x, float y, float z,
+                                             const float* g, float& pot, float& ax, float& ay,
+                                             float& az) {
+  const float x2 = x * x, y2 = y * y, z2 = z * z;
+  const float fxx = x2 - z2, fyy = y2 - z2;
+  const float x_2 = x + x, y_2 = y + y;
+  const float fxy = x_2 * y, fxz = x_2 * z, fyz = y_2 * z;
+  const float fxxx = x * __builtin_fmaf(-3.0f, z2, x2), fyyy = y * __builtin_fmaf(-3.0f, z2, y2);
+  const float fxyy = (3.0f * x) * fyy, fxxy = (3.0f * y) * fxx;
+  const float fxxz = z * __builtin_fmaf(3.0f, x2, -z2), fyyz = z * __builtin_fmaf(3.0f, y2, -z2);
+  const float fxyz = (3.0f * z) * fxy;
+  const float v2x = Q.xx * x + Q.xy * y + Q.xz * z;
+  const float v2y = Q.xy * x + Q.yy * y + Q.yz * z;
+  const float v2z = Q.xz * x + Q.yz * y + Q.zz * z;
+  const float v3x = Q.xxx * fxx + Q.xyy * fyy + Q.xxy * fxy + Q.xxz * fxz + Q.xyz * fyz;
+  const float v3y = Q.xyy * fxy + Q.xxy * fxx + Q.yyy * fyy + Q.yyz * fyz + Q.xyz * fxz;
+  const float v3z = Q.xxz * fxx + Q.yyz * fyy + Q.xyz * fxy + Q.q3a * fxz + Q.q3b * fyz;
+  const float v4x = Q.xxxx * fxxx + Q.xxyy * fxyy + Q.xxxy * fxxy + Q.xyyy * fyyy +
+                    Q.xxxz * fxxz + Q.xyyz * fyyz + Q.xxyz * fxyz;
+  const float v4y = Q.yyyy * fyyy + Q.xxyy * fxxy + Q.xxxy * fxxx + Q.xyyy * fxyy +
+                    Q.xyyz * fxyz + Q.xxyz * fxxz + Q.yyyz * fyyz;
+  const float v4z = Q.xxxz * fxxx + Q.xyyz * fxyy + Q.xxyz * fxxy + Q.yyyz * fyyy + Q.q4a * fxxz +
+                    Q.q4b * fyyz + Q.q4c * fxyz;
+  const float p2 = v2x * x + v2y * y + v2z * z;
+  const float p3 = v3x * x + v3y * y + v3z * z;
+  const float p4 = v4x * x + v4y * y + v4z * z;
+  pot = -(g[0] * Q.m + g[2] * p2 + g[3] * p3 + g[4] * p4);
+  const float ta = g[1] * Q.m + g[3] * p2 + g[4] * p3 + g[5] * p4;
+  const float c2 = 2.0f * g[2], c3 = 3.0f * g[3], c4 = 4.0f * g[4];
+  ax = c2 * v2x + c3 * v3x + c4 * v4x - ta * x;
+  ay = c2 * v2y + c3 * v3y + c4 * v4y - ta * y;
+  az = c2 * v2z + c3 * v3z + c4 * v4z - ta * z;
+}
+
+// radial32 with the error functions of x = alpha r >= 1 (all but a few
+// particles near a replica's copy of the root centre) from the exponential
+// the recursion needs anyway: erfc(x) = e^(-x^2) P(t), t = 1 / (1 + x / 2),
+// -erf = erfc - 1. P: degree-7 least-maximum fit of erfc(x) e^(x^2) on
+// 0.98 <= x <= 6.3 (own fit, relative error 1e-8; below that range's end
+// e^(-x^2) is zero to FP32). With e^(-x^2) from the unrounded x^2 the
+// relative error of erfc is at most 3.4e-7 for x <= 6.2, where erfcf of the
+// rounded x gives 6.5e-6, at a third of its instructions.
+__device__ __forceinline__ void radial32_fast(float r2, float hole, float alpha, float alpha2,
+                                              float ka, float inner2, float* g) {
+  const float dir = rsqrtf(r2), ir2 = dir * dir;
+  const float x = alpha * (r2 * dir);
+  if (r2 < inner2 || x < 1.0f) {
+    radial32(r2, hole != 0.0f, alpha, alpha2, ka, inner2, g);
+    return;
+  }
+  const float ex = expf(-alpha2 * r2);
+  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.5f, x, 1.0f));
+  float pt = 1.008342766e-01f;
+  pt = __builtin_fmaf(pt, t, -4.093811133e-01f);
+  pt = __builtin_fmaf(pt, t, 4.758980659e-01f);
+  pt = __builtin_fmaf(pt, t, -3.587170541e-02f);
+  pt = __builtin_fmaf(pt, t, 3.166909518e-01f);
+  pt = __builtin_fmaf(pt, t, 2.681522595e-01f);
+  pt = __builtin_fmaf(pt, t, 2.836491832e-01f);
+  pt = __builtin_fmaf(pt, t, -7.436778299e-05f);
+  g[0] = __builtin_fmaf(ex, pt, -hole) * dir;
+  const float e = ka * ex * ir2;
+  float s = 1.0f;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    g[k + 1] = (2 * k + 1) * g[k] * ir2 + s * e;
+    s *= 2 * alpha2;
+  }
+}
+
+__global__ __launch_bounds__(kEwBlock) __attribute__((amdgpu_waves_per_eu(5))) void ewald_kernel(const CompactPartData* parts,
                                                          VariablePartData* vars,
                                                          const int* markers, int first, int n,
                                                          const EwtData* ewt, const double* pos64,
@@ -39,16 +148,16 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
   extern __shared__ float4 sh[];
   // lattice offsets (n L, hole flag) that some particle of the wavefront needs
   __shared__ float4 cand[kEwBlock / kWave][kEwMaxCand];
-  __shared__ int ncand[kEwBlock / kWave];
+  __shared__ int lattice[kEwMaxCand];
 
   // the same table as weights on the cube |h_i| <= kEwCube (zero off the table)
   __shared__ float2 cube[kEwCubeN];
-  __shared__ int n_outside;
+  __shared__ int n_outside, n_uneven;
 
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
   const float kscale = (float)(p.L / (2.0 * M_PI));  // k -> integer h
   for (int i = tid; i < kEwCubeN; i += kEwBlock) cube[i] = make_float2(0.0f, 0.0f);
-  if (tid == 0) n_outside = 0;
+  if (tid == 0) n_outside = n_uneven = 0;
   __syncthreads();
   for (int i = tid; i < p.nH; i += kEwBlock) {
     EwtData e = ewt[i];
@@ -62,6 +171,22 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
     } else {
       atomicAdd(&n_outside, 1);
     }
+  }
+
+  // hC is even in h and hS odd (Ewald.cpp:359-381), so h and -h give the same
+  // term: with a table that holds both, the cube's upper half is doubled and
+  // the lower one cleared (and its planes skipped); any other table is kept
+  __syncthreads();
+  if (tid < kEwCubeN / 2) {
+    const float2 u = cube[tid], v = cube[kEwCubeN - 1 - tid];
+    if (u.x != v.x || u.y != -v.y) atomicAdd(&n_uneven, 1);
+  }
+  __syncthreads();
+  const bool even = n_uneven == 0;
+  if (even && tid < kEwCubeN / 2) {
+    const float2 v = cube[kEwCubeN - 1 - tid];
+    cube[kEwCubeN - 1 - tid] = make_float2(2.0f * v.x, 2.0f * v.y);
+    cube[tid] = make_float2(0.0f, 0.0f);
   }
 
   // root centre of mass, k = 0 term and moments: from the device root record
@@ -92,52 +217,47 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
       lo[k] = fminf(lo[k], __shfl_xor(lo[k], m, kWave));
       hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], m, kWave));
     }
+  // the lattice vectors, found once for the block: n + 3 in bytes, bit 24 hole
   const int W = 2 * p.nEwReps + 1, NC = W * W * W;
-  const float Lf = (float)p.L, cut2f = (float)p.cut2;
-  if (lane == 0) ncand[wv] = 0;
-  __syncthreads();
-  for (int c0 = 0; c0 < NC; c0 += kWave) {
-    int c = c0 + lane;
-    bool need = false;
-    if (c < NC) {
-      int ix = c / (W * W) - p.nEwReps, iy = (c / W) % W - p.nEwReps, iz = c % W - p.nEwReps;
-      bool hole = abs(ix) <= p.nReps && abs(iy) <= p.nReps && abs(iz) <= p.nReps;
-      bool centre = ix == 0 && iy == 0 && iz == 0;
-      int iv[3] = {ix, iy, iz};
-      float d2 = 0.f;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        float l = lo[k] + iv[k] * Lf, h = hi[k] + iv[k] * Lf;
-        float e = l > 0.f ? l : (h < 0.f ? -h : 0.f);
-        d2 += e * e;
-      }
-      // slack for FP32 rounding of the bound; the per-particle test is exact
-      need = !centre && (hole || d2 <= cut2f * 1.0001f + 1e-6f * Lf * Lf);
-    }
-    unsigned long long mask = __ballot(need);
-    int before = __popcll(mask & ((1ull << lane) - 1ull));
-    if (need) {
-      int ix = c / (W * W) - p.nEwReps, iy = (c / W) % W - p.nEwReps, iz = c % W - p.nEwReps;
-      bool hole = abs(ix) <= p.nReps && abs(iy) <= p.nReps && abs(iz) <= p.nReps;
-      cand[wv][ncand[wv] + before] = make_float4(ix * Lf, iy * Lf, iz * Lf, hole ? 1.0f : 0.0f);
-    }
-    __syncthreads();
-    if (lane == 0) ncand[wv] += __popcll(mask);
-    __syncthreads();
+  for (int c = tid; c < NC; c += kEwBlock) {
+    const int ix = c / (W * W) - p.nEwReps, iy = (c / W) % W - p.nEwReps, iz = c % W - p.nEwReps;
+    const bool hole = abs(ix) <= p.nReps && abs(iy) <= p.nReps && abs(iz) <= p.nReps;
+    lattice[c] = (ix + 3) | ((iy + 3) << 8) | ((iz + 3) << 16) | ((int)hole << 24);
   }
-  const int nc = ncand[wv];
+  const float Lf = (float)p.L, cut2f = (float)p.cut2;
+  __syncthreads();
+  // those that some particle of the wavefront needs, compacted
+  int nc = 0;
+  for (int c0 = 0; c0 < NC; c0 += kWave) {
+    const int c = c0 + lane;
+    const int v = lattice[min(c, NC - 1)];
+    const float n[3] = {(float)((v & 255) - 3) * Lf, (float)(((v >> 8) & 255) - 3) * Lf,
+                        (float)(((v >> 16) & 255) - 3) * Lf};
+    const bool hole = (v >> 24) != 0, centre = (v & 0xffffff) == 0x030303;
+    float d2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float l = lo[k] + n[k], h = hi[k] + n[k];
+      const float e = l > 0.f ? l : (h < 0.f ? -h : 0.f);
+      d2 += e * e;
+    }
+    // slack for FP32 rounding of the bound; the per-particle test is exact
+    const bool need = c < NC && !centre && (hole || d2 <= cut2f * 1.0001f + 1e-6f * Lf * Lf);
+    const unsigned long long mask = __ballot(need);
+    if (need)
+      cand[wv][nc + __popcll(mask & ((1ull << lane) - 1ull))] =
+          make_float4(n[0], n[1], n[2], hole ? 1.0f : 0.0f);
+    nc += __popcll(mask);
+  }
+  __syncthreads();
 
   Mom22<double> Qd;
-  Mom22<float> Qf;
   {
     double* qd = &Qd.m;
-    float* qf = &Qf.m;
 #pragma unroll
-    for (int k = 0; k < 22; ++k) {
-      qd[k] = root ? root[4 + k] : p.q[k];
-      qf[k] = (float)qd[k];
-    }
+    for (int k = 0; k < 22; ++k) qd[k] = root ? root[4 + k] : p.q[k];
   }
+  const EwaldMom32 Qf = ewald_mom32(Qd);
   double pot = mk1, ax = 0, ay = 0, az = 0;
   // central replica in FP64
   {
@@ -150,14 +270,13 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
               inner2 = (float)p.inner2, cut2 = (float)p.cut2;
   for (int k = 0; k < nc; ++k) {
     const float4 cv = cand[wv][k];
-    const bool hole = cv.w != 0.0f;
     float x = fx + cv.x, y = fy + cv.y, z = fz + cv.z;
     float r2 = x * x + y * y + z * z;
-    if (r2 > cut2 && !hole) continue;
+    if (r2 > cut2 && cv.w == 0.0f) continue;
     float g[6];
-    radial32(r2, hole, alpha, alpha2, ka, inner2, g);
-    float tp = 0.f, tx = 0.f, ty = 0.f, tz = 0.f;
-    ewald_term<float>(Qf, x, y, z, g, tp, tx, ty, tz);
+    radial32_fast(r2, cv.w, alpha, alpha2, ka, inner2, g);
+    float tp, tx, ty, tz;
+    ewald_term32(Qf, x, y, z, g, tp, tx, ty, tz);
     pot += tp;
     ax += tx;
     ay += ty;
@@ -176,14 +295,16 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
     sincospif(2.0f * ux, &e1x.y, &e1x.x);
     axis_powers(uy, ey);
     axis_powers(uz, ez);
-    float2 ex = cpow_neg(e1x);  // e^(-2 pi i kEwCube u_x)
+    const int hx0 = even ? 0 : -kEwCube;
+    float2 ex = even ? make_float2(1.0f, 0.0f) : cpow_neg(e1x);  // e^(2 pi i hx0 u_x)
     const float kf = (float)(2.0 * M_PI / p.L);
-    for (int hx = -kEwCube; hx <= kEwCube; ++hx) {
-      KahanF sp, sx, sy, sz;
+    for (int hx = hx0; hx <= kEwCube; ++hx) {
+      KahanF sp, st, sy, sz;
       const float2* cw = cube + (hx + kEwCube) * kEwCubeW * kEwCubeW;
 #pragma unroll
       for (int hy = -kEwCube; hy <= kEwCube; ++hy) {
         const float2 exy = cmul(ex, ey[hy + kEwCube]);
+        KahanF row;  // sum of t at this hy
 #pragma unroll
         for (int hz = -kEwCube; hz <= kEwCube; ++hz) {
           const float2 wgt = cw[(hy + kEwCube) * kEwCubeW + hz + kEwCube];
@@ -191,14 +312,19 @@ __global__ __launch_bounds__(kEwBlock) void ewald_kernel(const CompactPartData* 
             const float2 e = cmul(exy, ez[hz + kEwCube]);
             sp.add(wgt.x * e.x + wgt.y * e.y);
             const float t = wgt.x * e.y - wgt.y * e.x;
-            sx.add((float)hx * t);
-            sy.add((float)hy * t);
-            sz.add((float)hz * t);
+            row.add(t);
+            if (hz != 0) sz.add((float)hz * t);
           }
+        }
+        st.add(row.s);
+        st.c += row.c;
+        if (hy != 0) {
+          sy.add((float)hy * row.s);
+          sy.c += (float)hy * row.c;
         }
       }
       pot += (double)sp.s - (double)sp.c;
-      ax += (double)kf * ((double)sx.s - (double)sx.c);
+      ax += (double)kf * (double)hx * ((double)st.s - (double)st.c);
       ay += (double)kf * ((double)sy.s - (double)sy.c);
       az += (double)kf * ((double)sz.s - (double)sz.c);
       ex = cmul(ex, e1x);
