@@ -3,10 +3,11 @@
 //
 // The per-bucket kernels (gravity.hip) follow ChaNGa's one-launch-per-list
 // pattern (nodeGravityComputation / particleGravityComputation,
-// HostCUDA.cu:1008-1205, 1565-1751). Here one wavefront takes a bucket from a
+// HostCUDA.cu:1008-1205, 1565-1751). Here a workgroup takes a bucket from a
 // work queue, runs its cell list and then its particle list into the same
 // FP64 accumulators (the chunk loops of gravity_body.h), and updates the
-// bucket's VariablePartData once.
+// bucket's VariablePartData once. A workgroup is one wavefront, or, where
+// there are few buckets, several that share the lists (Team).
 //
 // Work queues. Buckets are cut into 8 contiguous ranges of equal estimated
 // cost, one per XCD, so that the waves of one XCD (workgroup id mod 8) share
@@ -61,12 +62,14 @@ struct BatchLds {
 // KMAX 1: one target per lane; 3: one to three, chosen per chunk by its size
 // (targets_per_lane). REC: cells from the 128-byte cell records.
 template <bool PRECISE, int KIND, int PCT, int PPT, int KMAX, bool REC>
-__device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane, float4* lds) {
+__device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane, const Team& team,
+                                             float4* lds_all) {
   const int pcs = a.pc.marks[b], pce = a.pc.marks[b + 1];
   const int pps = a.pp.marks[b], ppe = a.pp.marks[b + 1];
   const int bstart = a.pc.starts[b], n = a.pc.sizes[b];
   double cx0, cy0, cz0;
   bucket_centre<PRECISE>(a.pc.tpos64, bstart, n, cx0, cy0, cz0);
+  float4* lds = lds_all + team.wave * BatchLds<PCT, PPT>::f4;
   PpFwdLds<PPT>& s = *reinterpret_cast<PpFwdLds<PPT>*>(lds);
   for (int t0 = 0; t0 < n; t0 += kWave) {
     const int nt = min(kWave, n - t0);
@@ -78,19 +81,24 @@ __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane
       Acc64 acc[K];
 #pragma unroll
       for (int j = 0; j < K; ++j) acc[j] = {0.0, 0.0, 0.0, 0.0, 0.0f};
-      pc_cells<PRECISE, PCT, true, K, REC>(a.pc, pcs, pce, cx0, cy0, cz0, t, l, lds, acc);
-      pp_sources<PRECISE, KIND, PPT, true, K>(a.pp, pps, ppe, cx0, cy0, cz0, t, l, s, acc);
-      reduce_store<K>(lds, l, acc, a.pc.vars + bstart + t0);
+      pc_cells<PRECISE, PCT, true, K, REC>(a.pc, team.share(pcs, pce), team.share_end(pcs, pce),
+                                           cx0, cy0, cz0, t, l, lds, acc);
+      pp_sources<PRECISE, KIND, PPT, true, K>(a.pp, team.share(pps, ppe), team.share_end(pps, ppe),
+                                              cx0, cy0, cz0, t, l, s, acc);
+      reduce_store<K>(reinterpret_cast<char*>(lds_all),
+                      BatchLds<PCT, PPT>::f4 * sizeof(float4), team, l, acc,
+                      a.pc.vars + bstart + t0);
     };
     if constexpr (KMAX == 1) chunk(KTag<1>());
     else with_targets_per_lane(nt, chunk);
   }
 }
 
-// Persistent kernel: one wavefront per workgroup; runs until every queue is
-// exhausted. Each wave visits the 8 queues once, starting at its own XCD's,
-// and stays on a queue until a claim comes back past its end, so every wave
-// exits after finitely many claims and no wave waits on another.
+// Persistent kernel: one bucket per workgroup at a time; runs until every
+// queue is exhausted. Each workgroup visits the 8 queues once, starting at its
+// own XCD's, and stays on a queue until a claim comes back past its end, so
+// every one exits after finitely many claims and none waits on another; all
+// wavefronts of a workgroup see the same claim.
 // Four wavefronts per SIMD (128 VGPRs), because the FP32 VALU issues the
 // force loops faster with four than with three (gravity_body.h: pc_cells).
 // KMAX 1 holds one chunk loop and does not spill: on a sparse rung (one to
@@ -99,16 +107,24 @@ __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane
 // 28 to 42 registers around the tiles; on the dense 2^22 halos, where the
 // shared LDS reads weigh more, KMAX 3 measured 9.13 ms against 9.92.
 template <bool PRECISE, int KIND, int PCT, int PPT, int KMAX, bool REC>
-__global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(BatchArgs a) {
-  __shared__ float4 lds[BatchLds<PCT, PPT>::f4];
-  const int lane = threadIdx.x;
+__global__ __launch_bounds__(kWave * kTeamWaves) __attribute__((amdgpu_waves_per_eu(4))) void
+batch_kernel(BatchArgs a) {
+  extern __shared__ float4 lds[];  // BatchLds<PCT, PPT>::f4 per wavefront
+  const int lane = threadIdx.x & (kWave - 1);
+  const Team team = block_team();
   const int* qbeg = a.queue;
   const int* ids = a.queue + kQueueHdr;
   int q = blockIdx.x % kNumXcd;
   for (int tried = 0; tried < kNumXcd;) {
     int k = 0;
-    if (lane == 0) k = atomicAdd(a.counters + q * kCounterStride, a.grab);
+    if (threadIdx.x == 0) k = atomicAdd(a.counters + q * kCounterStride, a.grab);
+    if (team.waves > 1) {
+      int* claimed = reinterpret_cast<int*>(lds);  // free between buckets
+      if (threadIdx.x == 0) *claimed = k;
+      __syncthreads();
+      k = *claimed;
+      __syncthreads();
+    }
     k = __builtin_amdgcn_readfirstlane(k);
     const int q0 = qbeg[q], qn = qbeg[q + 1] - q0;
     if (k >= qn) {
@@ -118,7 +134,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(BatchArgs a) {
     }
     const int kend = min(k + a.grab, qn);
     for (; k < kend; ++k)
-      batch_bucket<PRECISE, KIND, PCT, PPT, KMAX, REC>(a, ids[q0 + k], lane, lds);
+      batch_bucket<PRECISE, KIND, PCT, PPT, KMAX, REC>(a, ids[q0 + k], lane, team, lds);
   }
 }
 
@@ -152,22 +168,33 @@ __global__ void bucket_cost_kernel(ChangaGravityLaunch pc, ChangaGravityLaunch p
 
 using BatchFn = void (*)(BatchArgs);
 
+// the kernel of a set of options and its LDS per wavefront
+struct BatchKernel {
+  BatchFn fn;
+  size_t lds;
+};
+
+template <bool PR, int KIND, int PCT, int PPT, int KM, bool REC>
+static BatchKernel batch_of() {
+  return {batch_kernel<PR, KIND, PCT, PPT, KM, REC>, BatchLds<PCT, PPT>::f4 * sizeof(float4)};
+}
+
 template <bool PR, int KIND, int KM, bool REC>
-static BatchFn pick_tiles(int pct, int ppt) {
+static BatchKernel pick_tiles(int pct, int ppt) {
   if (pct == 32)
-    return ppt == 128 ? batch_kernel<PR, KIND, 32, 128, KM, REC>
-                      : batch_kernel<PR, KIND, 32, 256, KM, REC>;
-  return ppt == 128 ? batch_kernel<PR, KIND, 64, 128, KM, REC>
-                    : batch_kernel<PR, KIND, 64, 256, KM, REC>;
+    return ppt == 128 ? batch_of<PR, KIND, 32, 128, KM, REC>()
+                      : batch_of<PR, KIND, 32, 256, KM, REC>();
+  return ppt == 128 ? batch_of<PR, KIND, 64, 128, KM, REC>()
+                    : batch_of<PR, KIND, 64, 256, KM, REC>();
 }
 
 template <bool PR, int KIND, bool REC>
-static BatchFn pick_kmax(int pct, int ppt, int kmax) {
+static BatchKernel pick_kmax(int pct, int ppt, int kmax) {
   return kmax == 1 ? pick_tiles<PR, KIND, 1, REC>(pct, ppt) : pick_tiles<PR, KIND, 3, REC>(pct, ppt);
 }
 
 template <bool REC>
-static BatchFn pick_rec(bool pr, int kind, const ChangaBatchOptions& o) {
+static BatchKernel pick_rec(bool pr, int kind, const ChangaBatchOptions& o) {
   const int pct = o.pcTile, ppt = o.ppTile, km = o.targetsPerLane;
   if (pr)
     return kind ? pick_kmax<true, 1, REC>(pct, ppt, km) : pick_kmax<true, 0, REC>(pct, ppt, km);
@@ -175,7 +202,7 @@ static BatchFn pick_rec(bool pr, int kind, const ChangaBatchOptions& o) {
 }
 
 // the kernel for these options; with cell records when the launch has them
-static BatchFn pick(bool pr, int kind, const ChangaBatchOptions& o, bool rec) {
+static BatchKernel pick(bool pr, int kind, const ChangaBatchOptions& o, bool rec) {
   return rec ? pick_rec<true>(pr, kind, o) : pick_rec<false>(pr, kind, o);
 }
 
@@ -198,14 +225,23 @@ struct ChangaBatchPlan {
 
 namespace {
 
-// Resident workgroups of the persistent kernel on the whole device; -1 on error.
-int grid_for(BatchFn fn) {
+// Wavefronts per bucket of the persistent kernel. us with 1 / 2 / 4 (medians
+// over the tuned configurations): 541 buckets 88 / 50 / 34, 2,074 90 / 64 / 59,
+// 4,051 114 / 94 / 95, 7,985 174 / 161 / 172, 12,004 603 / 599 / 642, 15,948
+// 314 / 309 / 341, 20,185 of a sparse rung 188 / 199 / 265.
+int batch_waves(int buckets) { return team_waves(buckets, 2048, 8192); }
+
+// Workgroups of the persistent kernel over this many buckets: those resident
+// on the whole device, but no more than there are buckets to claim. -1 on error.
+int grid_for(const BatchKernel& k, int buckets) {
+  const int waves = batch_waves(buckets);
   int dev = 0, ncu = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)fn, kWave, 0) != hipSuccess)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k.fn, kWave * waves,
+                                                   k.lds * waves) != hipSuccess)
     return -1;
-  return ncu * std::max(per, 1);
+  return std::min(ncu * std::max(per, 1), std::max(buckets, 1));
 }
 
 // Enqueue one batched evaluation with the plan's chosen configuration.
@@ -218,11 +254,13 @@ int enqueue(const ChangaBatchPlan* p, const BatchArgs& args, const ChangaBatchOp
   hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(kNumXcd * kCounterStride), 0, s,
                      args.counters);
   CGPU_CHECK(hipGetLastError());
-  BatchFn fn = pick(p->precise, p->kind, o, o.cellSource == 1);
+  const BatchKernel k = pick(p->precise, p->kind, o, o.cellSource == 1);
+  const int waves = batch_waves(args.pc.numBuckets);
   BatchArgs a = args;
   a.grab = o.listsPerGrab;
   void* kargs[] = {&a};
-  CGPU_CHECK(hipLaunchKernel((const void*)fn, dim3(grid), dim3(kWave), kargs, 0, s));
+  CGPU_CHECK(hipLaunchKernel((const void*)k.fn, dim3(grid), dim3(kWave * waves), kargs,
+                             k.lds * waves, s));
   return 0;
 }
 
@@ -386,7 +424,7 @@ extern "C" int changaBatchPlanCreate(const ChangaGravityLaunch* cells,
       a.pc.vars = scratch;
       a.pp.vars = scratch;
       a.queue = d_q[c.order - 1];
-      const int grid = grid_for(pick(p->precise, p->kind, c, c.cellSource == 1));
+      const int grid = grid_for(pick(p->precise, p->kind, c, c.cellSource == 1), nb);
       if (grid <= 0) {
         e = hipErrorInvalidValue;
         return -1.0f;
@@ -487,7 +525,7 @@ extern "C" int changaBatchPlanCreate(const ChangaGravityLaunch* cells,
   p->args.queue = p->d_queue;
   p->args.grab = o.listsPerGrab;
   if (nb > 0) {
-    p->grid = grid_for(pick(p->precise, p->kind, o, o.cellSource == 1));
+    p->grid = grid_for(pick(p->precise, p->kind, o, o.cellSource == 1), nb);
     if (p->grid <= 0) return bail(fail("batch plan: occupancy", hipErrorInvalidValue, __FILE__,
                                        __LINE__));
     // capture reset (+ zeroing) + persistent kernel; every node is a kernel
@@ -710,8 +748,9 @@ extern "C" int changaBatchedGravityNoAlloc(const ChangaGravityLaunch* cells,
   if (int e = na_scratch(&dev, &ws)) return e;
   if (nb == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  const BatchFn fn = pick(pc.tpos64 != nullptr, pp.listKind, o, o.cellSource == 1);
-  const int grid = grid_for(fn);
+  const BatchKernel k = pick(pc.tpos64 != nullptr, pp.listKind, o, o.cellSource == 1);
+  const int waves = batch_waves(nb);
+  const int grid = grid_for(k, nb);
   if (grid <= 0)
     return fail("changaBatchedGravityNoAlloc: occupancy", hipErrorInvalidValue, __FILE__,
                 __LINE__);
@@ -742,6 +781,7 @@ extern "C" int changaBatchedGravityNoAlloc(const ChangaGravityLaunch* cells,
   a.counters = ws + kNaCounters;
   a.grab = o.listsPerGrab;
   void* kargs[] = {&a};
-  CGPU_CHECK(hipLaunchKernel((const void*)fn, dim3(grid), dim3(kWave), kargs, 0, s));
+  CGPU_CHECK(hipLaunchKernel((const void*)k.fn, dim3(grid), dim3(kWave * waves), kargs,
+                             k.lds * waves, s));
   return 0;
 }

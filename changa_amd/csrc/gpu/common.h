@@ -31,6 +31,15 @@ int fail(const char* what, hipError_t e, const char* file, int line);
     if (_e != hipSuccess) return cgpu::fail(#expr, _e, __FILE__, __LINE__); \
   } while (0)
 
+// Orders this wavefront's LDS accesses before against those after, for data
+// that only its own lanes exchange: a wavefront's LDS instructions execute in
+// order, so nothing has to wait (a workgroup barrier also waits for the
+// global loads in flight, and for the other wavefronts where there are any).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Replica offset of offsetID bits 22-30 (TreePiece.cpp:3631-3645;
 // ParallelGravity.h:2064-2073) as integer multiples of the period.
 __device__ __forceinline__ int off_x(int oid) { return ((oid >> 22) & 7) - 3; }

@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void fu
                                          lds, acc);
       pp_sources<true, 1, PPT, false, 1>(a.pp, rbase, rbase + nruns, cx0, cy0, cz0, t, l, ps,
                                          acc);
-      reduce_store<1>(lds, l, acc, a.pc.vars + bstart + t0);
+      reduce_store<1>(reinterpret_cast<char*>(lds), 0, {1, 0}, l, acc, a.pc.vars + bstart + t0);
     }
   }
 }

@@ -7,22 +7,32 @@
 
 namespace cgpu {
 
+// float4 of LDS per wavefront
+constexpr int kPcLds = (kPcTile + 1) * (kFwdRec / 4);
+constexpr int kPpLds = (sizeof(PpFwdLds<kPpTile>) + 15) / 16;
+static_assert(kPcLds * sizeof(float4) >= reduce_bytes<2>() &&
+                  kPpLds * sizeof(float4) >= reduce_bytes<3>(),
+              "reduction");
+
 // ---------------------------------------------------------------------------
-// Per-bucket particle-cell kernel: one 64-lane workgroup per bucket, buckets
-// mapped to XCDs in contiguous ranges (xcd_bucket).
+// Per-bucket particle-cell kernel: one workgroup per bucket, of one wavefront
+// or, in launches of few buckets, of several that share its list (Team);
+// buckets mapped to XCDs in contiguous ranges (xcd_bucket).
 // ---------------------------------------------------------------------------
 // REC: cells from the 128-byte cell records, else from the wire moments; in
 // tiles of 64 either way (records in tiles of 32: 128^3 box 2.34 ms against
 // 2.22, 256^3 box with a 10% rung 8.05 against 6.11). At most two targets
 // per lane: no spills at four wavefronts per SIMD.
 template <bool PRECISE, bool REC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pc_kernel(
-    ChangaGravityLaunch a) {
-  // staged tile; reused for the slot reduction at the end of each chunk
-  __shared__ float4 rec4[(kPcTile + 1) * (kFwdRec / 4)];
-  static_assert(sizeof(rec4) >= reduce_bytes<2>(), "reduction");
+__global__ __launch_bounds__(kWave * kTeamWaves) __attribute__((amdgpu_waves_per_eu(4))) void
+pc_kernel(ChangaGravityLaunch a) {
+  // staged tile of each wavefront; reused for the slot reduction at the end
+  // of each chunk
+  extern __shared__ float4 lds[];
+  const int lane = threadIdx.x & (kWave - 1);
+  const Team team = block_team();
+  float4* rec4 = lds + team.wave * kPcLds;
 
-  const int lane = threadIdx.x;
   const int b = xcd_bucket(blockIdx.x, a.numBuckets);
   const int start = a.marks[b], end = a.marks[b + 1];
   const int bstart = a.starts[b], n = a.sizes[b];
@@ -39,8 +49,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pc
       Acc64 acc[K];
 #pragma unroll
       for (int j = 0; j < K; ++j) acc[j] = {0.0, 0.0, 0.0, 0.0, 0.0f};
-      pc_cells<PRECISE, kPcTile, true, K, REC>(a, start, end, cx0, cy0, cz0, t, l, rec4, acc);
-      reduce_store<K>(rec4, l, acc, a.vars + bstart + t0);
+      pc_cells<PRECISE, kPcTile, true, K, REC>(a, team.share(start, end),
+                                               team.share_end(start, end), cx0, cy0, cz0, t, l,
+                                               rec4, acc);
+      reduce_store<K>(reinterpret_cast<char*>(lds), kPcLds * sizeof(float4), team, l, acc,
+                      a.vars + bstart + t0);
     });
   }
 }
@@ -49,12 +62,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pc
 // Per-bucket particle-particle kernel (KIND: see pp_sources).
 // ---------------------------------------------------------------------------
 template <bool PRECISE, int KIND>
-__global__ __launch_bounds__(64) void pp_kernel(ChangaGravityLaunch a) {
-  // staged tiles; reused for the slot reduction at the end of each chunk
-  __shared__ PpFwdLds<kPpTile> s;
-  static_assert(sizeof(s) >= reduce_bytes<3>(), "reduction");
+__global__ __launch_bounds__(kWave * kTeamWaves) __attribute__((amdgpu_waves_per_eu(4))) void
+pp_kernel(ChangaGravityLaunch a) {
+  // staged tiles of each wavefront; reused for the slot reduction at the end
+  // of each chunk
+  extern __shared__ float4 lds[];
+  const int lane = threadIdx.x & (kWave - 1);
+  const Team team = block_team();
+  PpFwdLds<kPpTile>& s = *reinterpret_cast<PpFwdLds<kPpTile>*>(lds + team.wave * kPpLds);
 
-  const int lane = threadIdx.x;
   const int b = xcd_bucket(blockIdx.x, a.numBuckets);
   const int start = a.marks[b], end = a.marks[b + 1];
   const int bstart = a.starts[b], n = a.sizes[b];
@@ -71,8 +87,11 @@ __global__ __launch_bounds__(64) void pp_kernel(ChangaGravityLaunch a) {
       Acc64 acc[K];
 #pragma unroll
       for (int j = 0; j < K; ++j) acc[j] = {0.0, 0.0, 0.0, 0.0, 0.0f};
-      pp_sources<PRECISE, KIND, kPpTile, true, K>(a, start, end, cx0, cy0, cz0, t, l, s, acc);
-      reduce_store<K>(&s, l, acc, a.vars + bstart + t0);
+      pp_sources<PRECISE, KIND, kPpTile, true, K>(a, team.share(start, end),
+                                                  team.share_end(start, end), cx0, cy0, cz0, t, l,
+                                                  s, acc);
+      reduce_store<K>(reinterpret_cast<char*>(lds), kPpLds * sizeof(float4), team, l, acc,
+                      a.vars + bstart + t0);
     });
   }
 }
@@ -164,14 +183,14 @@ extern "C" int changaNodeGravity(const ChangaGravityLaunch* a, void* stream) {
     return fail("changaNodeGravity: cellRecords not 128-byte aligned", hipErrorInvalidValue,
                 __FILE__, __LINE__);
   hipStream_t s = (hipStream_t)stream;
-  const dim3 g(a->numBuckets), blk(kWave);
-  if (a->cellRecords) {
-    if (a->tpos64) hipLaunchKernelGGL((pc_kernel<true, true>), g, blk, 0, s, *a);
-    else hipLaunchKernelGGL((pc_kernel<false, true>), g, blk, 0, s, *a);
-  } else {
-    if (a->tpos64) hipLaunchKernelGGL((pc_kernel<true, false>), g, blk, 0, s, *a);
-    else hipLaunchKernelGGL((pc_kernel<false, false>), g, blk, 0, s, *a);
-  }
+  // us with 1 / 2 / 4 wavefronts per bucket: 541 buckets 18 / 12 / 11, 2,074
+  // 41 / 34 / 32, 7,985 136 / 129 / 136, 15,948 262 / 263 / 278, 20,185 of a
+  // sparse rung 109 / 129 / 178
+  const int waves = team_waves(a->numBuckets, 2048, 8192);
+  const auto kernel = a->cellRecords ? (a->tpos64 ? pc_kernel<true, true> : pc_kernel<false, true>)
+                                     : (a->tpos64 ? pc_kernel<true, false> : pc_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(a->numBuckets), dim3(kWave * waves),
+                     waves * kPcLds * sizeof(float4), s, *a);
   CGPU_CHECK(hipGetLastError());
   return 0;
 }
@@ -202,15 +221,15 @@ extern "C" int changaPartGravity(const ChangaGravityLaunch* a, void* stream) {
     return fail("changaPartGravity: precision form needs spos64", hipErrorInvalidValue, __FILE__,
                 __LINE__);
   hipStream_t s = (hipStream_t)stream;
-  dim3 g(a->numBuckets), blk(kWave);
-  bool pr = a->tpos64 != nullptr;
-  if (a->listKind == 0) {
-    if (pr) hipLaunchKernelGGL((pp_kernel<true, 0>), g, blk, 0, s, *a);
-    else hipLaunchKernelGGL((pp_kernel<false, 0>), g, blk, 0, s, *a);
-  } else {
-    if (pr) hipLaunchKernelGGL((pp_kernel<true, 1>), g, blk, 0, s, *a);
-    else hipLaunchKernelGGL((pp_kernel<false, 1>), g, blk, 0, s, *a);
-  }
+  // the lists are a third of the cells' in time: 541 buckets 23 / 17 / 13 us
+  // with 1 / 2 / 4 wavefronts per bucket, 2,074 25 / 23 / 25, 3,850 16 / 19 /
+  // 30, 7,985 43 / 52 / 72
+  const int waves = team_waves(a->numBuckets, 1024, 2048);
+  const bool pr = a->tpos64 != nullptr;
+  const auto kernel = a->listKind == 0 ? (pr ? pp_kernel<true, 0> : pp_kernel<false, 0>)
+                                       : (pr ? pp_kernel<true, 1> : pp_kernel<false, 1>);
+  hipLaunchKernelGGL(kernel, dim3(a->numBuckets), dim3(kWave * waves),
+                     waves * kPpLds * sizeof(float4), s, *a);
   CGPU_CHECK(hipGetLastError());
   return 0;
 }

@@ -391,7 +391,7 @@ __device__ __forceinline__ void stage_rec_tile(const RecTile<TILE>& f, int nc, i
   [&]<int... J>(std::integer_sequence<int, J...>) {
     ((dst[8 * J] = f.v[J]), ...);
   }(std::make_integer_sequence<int, TILE / 8>());
-  __syncthreads();
+  wave_sync();
   if (lane < nc) {
     float4* r = rec4 + lane;
     const float4 p0 = r[0], p1 = r[PS], p5 = r[5 * PS], p6 = r[6 * PS], p7 = r[7 * PS];
@@ -407,7 +407,7 @@ __device__ __forceinline__ void stage_rec_tile(const RecTile<TILE>& f, int nc, i
     r[0] = make_float4(x, y, z, q4a);
     r[PS] = make_float4(q4b, q4c, p1.z, (oid & CHANGA_ILCELL_SOFTENED) ? p1.w : -1.0f);
   }
-  __syncthreads();
+  wave_sync();
 }
 
 
@@ -539,23 +539,54 @@ __device__ __forceinline__ void load_targets(const ChangaGravityLaunch& a, int t
   }
 }
 
-// Doubles of LDS the slot reduction of K targets per lane needs (the floats
-// of dtGrav included).
+// Bytes of LDS the slot reduction of K targets per lane needs.
 template <int K>
 constexpr size_t reduce_bytes() {
   return (size_t)K * kWave * (4 * sizeof(double) + sizeof(float));
+}
+
+// Wavefronts that share one bucket's lists, its blocks' size in wavefronts
+// and this one's number. Each takes a contiguous share of a list.
+struct Team {
+  int waves, wave;
+  __device__ __forceinline__ int share(int start, int end) const {  // start of this one's share
+    return start + (int)((long long)(end - start) * wave / waves);
+  }
+  __device__ __forceinline__ int share_end(int start, int end) const {
+    return start + (int)((long long)(end - start) * (wave + 1) / waves);
+  }
+};
+
+constexpr int kTeamWaves = 4;
+
+// The team of a block that is one (blockDim.x: its wavefronts x 64).
+__device__ __forceinline__ Team block_team() {
+  return {(int)(blockDim.x / kWave), (int)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave)};
+}
+
+// Wavefronts per bucket for a launch over this many buckets: kTeamWaves up to
+// `four` of them, two up to `two`, else one. A bucket's lists are a serial
+// chain of tiles for one wavefront, and the card holds 4,096 wavefronts at
+// four per SIMD: with fewer buckets than that a launch waits for its longest
+// list, and splitting the lists both shortens the chain and fills the card;
+// with more the shares of a tile cost staging and a join per bucket.
+static inline int team_waves(int buckets, int four, int two) {
+  return buckets <= four ? kTeamWaves : buckets <= two ? 2 : 1;
 }
 
 // Slot reduction in a fixed order and the += into the result array (+= for
 // a and phi, max for dtGrav): every lane stores the sums of its places, the
 // slots are added pairwise (slot s += slot s + h, h = ceil(n / 2), while
 // n > 1 slots are left: log2(nslot) rounds, all lanes at once), then lane
-// i < nt adds target i's total, now in slot 0. lds: reduce_bytes<K>().
+// i < nt of the team's first wavefront adds target i's totals, now in slot 0
+// of each wavefront. lds: reduce_bytes<K>() per wavefront, `stride` bytes
+// apart; this one's is the wave-th.
 template <int K>
-__device__ __forceinline__ void reduce_store(void* lds, const Lanes& l, const Acc64 (&acc)[K],
+__device__ __forceinline__ void reduce_store(char* lds, size_t stride, const Team& team,
+                                             const Lanes& l, const Acc64 (&acc)[K],
                                              VariablePartData* out) {
   constexpr int W = K * kWave;
-  double* red = static_cast<double*>(lds);
+  double* red = reinterpret_cast<double*>(lds + team.wave * stride);
   float* redi = reinterpret_cast<float*>(red + 4 * W);
 #pragma unroll
   for (int j = 0; j < K; ++j) {
@@ -567,7 +598,7 @@ __device__ __forceinline__ void reduce_store(void* lds, const Lanes& l, const Ac
     red[3 * W + i] = v ? acc[j].pot : 0.0;
     redi[i] = v ? acc[j].idt : 0.0f;
   }
-  __syncthreads();
+  wave_sync();
   for (int n = l.nslot; n > 1;) {
     const int h = (n + 1) >> 1;
     if (l.slot < n - h) {
@@ -583,19 +614,31 @@ __device__ __forceinline__ void reduce_store(void* lds, const Lanes& l, const Ac
       }
     }
     n = h;
-    __syncthreads();
+    wave_sync();
   }
-  if (l.lane < l.nt) {
+  if (team.waves > 1) __syncthreads();
+  if (l.lane < l.nt && team.wave == 0) {
     const int j = l.lane / l.ng, i = j * kWave + (l.lane - j * l.ng);
+    double ax = red[i], ay = red[W + i], az = red[2 * W + i], pot = red[3 * W + i];
+    float idt = redi[i];
+    for (int w = 1; w < team.waves; ++w) {
+      const double* r = reinterpret_cast<const double*>(lds + w * stride);
+      ax += r[i];
+      ay += r[W + i];
+      az += r[2 * W + i];
+      pot += r[3 * W + i];
+      idt = fmaxf(idt, reinterpret_cast<const float*>(r + 4 * W)[i]);
+    }
     VariablePartData v = out[l.lane];
-    v.a.x += (float)red[i];
-    v.a.y += (float)red[W + i];
-    v.a.z += (float)red[2 * W + i];
-    v.potential += (float)red[3 * W + i];
-    v.dtGrav = fmaxf(v.dtGrav, redi[i]);
+    v.a.x += (float)ax;
+    v.a.y += (float)ay;
+    v.a.z += (float)az;
+    v.potential += (float)pot;
+    v.dtGrav = fmaxf(v.dtGrav, idt);
     out[l.lane] = v;
   }
-  __syncthreads();
+  if (team.waves > 1) __syncthreads();
+  else wave_sync();
 }
 
 // Cells [start, end) of a.list onto the chunk's targets. Tiles of TILE <= 64
@@ -658,7 +701,7 @@ __device__ __forceinline__ void pc_cells(const ChangaGravityLaunch& a, int start
       stage_rec_tile<PRECISE, TILE, PS>(rt, nc, l.lane, oid, L, shifted, cx0, cy0, cz0, rec4);
     } else {
       if (mine) stage_cell_fwd<PRECISE, PS>(a, w, L, shifted, cx0, cy0, cz0, rec4 + l.lane);
-      __syncthreads();
+      wave_sync();
     }
     if (l.live) {
       Acc32 A[K];
@@ -705,7 +748,7 @@ __device__ __forceinline__ void pc_cells(const ChangaGravityLaunch& a, int start
         acc[j].idt = A[j].idt;
       }
     }
-    __syncthreads();
+    wave_sync();
   }
 }
 
@@ -914,7 +957,7 @@ __device__ __forceinline__ void pp_source_tiles(const ChangaGravityLaunch& a, in
         const int ns = min(TILE, total - sb);
         const int j1 = min(incl, sb + ns);
         for (int j = max(begin, sb); j < j1; ++j) map[j - sb] = make_int2(first + (j - begin), oid);
-        __syncthreads();
+        wave_sync();
         tile(ns, [&](int i) { return map[i]; });
       }
     }
@@ -989,7 +1032,7 @@ __device__ __forceinline__ void pp_sources(const ChangaGravityLaunch& a, int sta
     const int q = (nfar + l.nslot - 1) / l.nslot;
     for (int k = nfar + lane; k < l.nslot * q; k += kWave)
       s.rec[k] = make_float4(1e18f, 1e18f, 1e18f, 0.0f);
-    __syncthreads();
+    wave_sync();
     if (l.live) {
       Acc32 A[K];
 #pragma unroll
@@ -1024,7 +1067,7 @@ __device__ __forceinline__ void pp_sources(const ChangaGravityLaunch& a, int sta
         acc[j].idt = A[j].idt;
       }
     }
-    __syncthreads();
+    wave_sync();
   });
 }
 

@@ -342,7 +342,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void lt
                                                       0.0, 0.0, t, l, lds, acc);
         pp_sources<false, 1, kLtwPpTile, false, 1>(a.pp, rbase, rbase + nruns, 0.0, 0.0, 0.0, t,
                                                    l, ps, acc);
-        reduce_store<1>(lds, l, acc, a.pc.vars + t0);
+        reduce_store<1>(reinterpret_cast<char*>(lds), 0, {1, 0}, l, acc, a.pc.vars + t0);
       }
     }
   }
