@@ -15,17 +15,28 @@
 // softened cells, then particle runs (the layout ListCompute::stateReady
 // serializes, Compute.cpp:1735-1741, 1806).
 //
-// One lane per target bucket walks depth first, in the
-// host walk's order (replicas from (-R, -R, -R) to (R, R, R), z fastest;
-// the first child first), so the lists are the host walk's entry for entry.
+// One lane per target bucket, a wavefront per group of up to 64 consecutive
+// ones. The wavefront walks the union of its buckets' walks depth first, in
+// the host walk's order (replicas from (-R, -R, -R) to (R, R, R), z fastest;
+// the first child first), and a lane takes part in the nodes that its own
+// bucket's walk visits, so the lists are the host walk's entry for entry.
 // The nodes are read as 64-byte walk records and tested in FP64 with
 // contraction off (walk_rec.h), so every opening decision is the host's on
 // the same node geometry. Two passes: count (per bucket: hexadecapole cells,
 // softened cells, runs, source particles; it also writes the walk records and
 // the escape nodes that let a lane walk depth first without a stack),
-// then, after the caller allocated the lists, fill. (A wavefront-cooperative
-// count walk, one wavefront per bucket, measured slower: a lane per bucket
-// keeps 64 times more independent node loads in flight.)
+// then, after the caller allocated the lists, fill.
+//
+// The node is the same for the whole wavefront, so its record is one scalar
+// load and its tests run on scalar operands. With a walk of its own per lane
+// every step gathered 64 records of 64 bytes, and the texture pipe bounded
+// both passes. The union costs more steps (2,069 a wavefront of 64 in the
+// 128^3 box, about 1.6 times one bucket's), the time of a step is the
+// wavefront's own instructions, and 128^3 took 1.41 + 2.02 ms before, 1.24 +
+// 1.54 now. Loading the records of both possible next nodes ahead cost 40
+// more scalar instructions a step (1.49 + 1.50), through one vector load and
+// readlanes 1.84 + 1.92. (A wavefront's lanes on the nodes of one bucket,
+// the fused form's walk, measured slower too.)
 #include <rocprim/device/device_scan.hpp>
 
 #include "common.h"
@@ -36,8 +47,24 @@ namespace cgpu {
 constexpr int kWalkBlock = 64;
 constexpr int kEscPasses = 8;  // pointer-jumping passes (even): chains up to 2^8 > the tree depth
 
+// Buckets per wavefront: the largest power of two (up to 64) that leaves
+// 1,900 wavefronts, about two per SIMD. More buckets share more of their
+// walks, fewer shorten each wavefront's chain of steps while the card has
+// room for more wavefronts. Count pass in us with 1 / 4 / 8 / 16 / 32 / 64
+// (and with a walk per lane): 541 buckets 177 / 208 / 227 / 269 / 340 / 406
+// (482), 7,985 - / 624 / 609 / 649 / 706 / 914 (980), 30,932 of a box - / 718
+// / 589 / 549 / 662 / 729 (862), 86,700 of a sparse rung - / 2,808 / 1,964 /
+// 1,565 / 1,552 / 1,818 (1,727), 126,534 - / 5,107 / 3,123 / 2,029 / 1,507 /
+// 1,309 (1,602).
+static int walk_group(int nb) {
+  int g = 1;
+  while (g < kWalkBlock && nb / 1900 >= 2 * g) g *= 2;
+  return g;
+}
+
 struct WalkArgs {
   int nb;
+  int group;   // buckets per wavefront (walk_group)
   int* nCell;  // count pass: cells (hexadecapole + softened) and runs per bucket
   int* nPart;
   const int* bucketNode;
@@ -55,59 +82,84 @@ struct WalkArgs {
   int* err;
 };
 
+// a walk record at a wave-uniform index: one scalar load of its cache line
+// (the records are written by an earlier launch)
+struct RecLine {
+  typedef int Line __attribute__((ext_vector_type(16)));
+  Line v;
+  __device__ __forceinline__ void load(const WalkRec* rec, int nd) {
+    v = *((const __attribute__((address_space(4))) Line*)(rec + nd));
+  }
+  __device__ __forceinline__ WalkRec get() const { return __builtin_bit_cast(WalkRec, v); }
+};
+
 // node record (node64): cm.xyz, radius, soft, mass, lo.xyz, hi.xyz, moments
 template <bool FILL>
 __global__ __launch_bounds__(kWalkBlock) void walk_kernel(WalkArgs a) {
-  // blocks of 64 consecutive buckets, each XCD taking a contiguous range of
-  // blocks so that its L2 holds the nodes near its buckets
-  const int b = xcd_bucket(blockIdx.x, gridDim.x) * kWalkBlock + threadIdx.x;
-  if (b >= a.nb) return;
+  // blocks of `group` consecutive buckets, each XCD taking a contiguous range
+  // of blocks so that its L2 holds the nodes near its buckets
+  const int b = xcd_bucket(blockIdx.x, gridDim.x) * a.group + threadIdx.x;
+  const bool live = (int)threadIdx.x < a.group && b < a.nb;
   double bg[12];
   {
-    const double* g = a.node64 + (size_t)a.bucketNode[b] * 34;
+    const double* g = a.node64 + (size_t)a.bucketNode[live ? b : a.nb - 1] * 34;
 #pragma unroll
     for (int k = 0; k < 12; ++k) bg[k] = g[k];
   }
   const double rb = 2.0 * bg[4];
   int nhex = 0, nsoft = 0, nruns = 0, nsrc = 0;
   int hpos = 0, spos = 0, ppos = 0;
-  if (FILL) {
+  if (FILL && live) {
     hpos = a.cellMarks[b];
     spos = a.softStart[b];
     ppos = a.partMarks[b];
   }
-  // depth first without a stack: an opened internal node continues with its
-  // first child; anything else continues with its escape node (the next node
-  // of the depth-first order after its subtree; -1 after the last)
   for (int x = -a.R; x <= a.R; ++x)
     for (int y = -a.R; y <= a.R; ++y)
       for (int z = -a.R; z <= a.R; ++z) {
         const int oid = ((x + 3) | ((y + 3) << 3) | ((z + 3) << 6)) << 22;
         const double ox = x * a.period, oy = y * a.period, oz = z * a.period;
-        int nd = 0;
-        while (nd >= 0) {
-          const WalkRec v = a.rec[nd];
-          const int next = v.link;  // the escape node
-          const int kind = walk_decide(v, bg, rb, ox, oy, oz);
-          if (kind == 2) {
-            if (FILL) a.cells[spos + nsoft] = {nd, oid | b | (int)0x80000000u};
-            ++nsoft;
-            nd = next;
-          } else if (kind == 1) {
-            if (FILL) a.cells[hpos + nhex] = {nd, oid | b};
-            ++nhex;
-            nd = next;
-          } else if (v.c0 < 0) {
-            if (FILL) a.parts[ppos + nruns] = {v.first, oid, v.count};
-            ++nruns;
-            nsrc += v.count;
-            nd = next;
-          } else {
+        int nd = live ? 0 : -2;  // this lane's next node
+        int cur = 0;             // the wavefront's
+        RecLine line;
+        line.load(a.rec, 0);
+        while (cur >= 0) {
+          const WalkRec v = line.get();
+          const bool here = nd == cur;
+          bool open = here, soft = false;
+          if (v.count > 6) {  // walk_decide, skipping what no lane needs
+#pragma clang fp contract(off)
+            const double c3[3] = {v.cx + ox, v.cy + oy, v.cz + oz};
+            const double dsq = walk_box_dsq(bg + 6, bg + 9, c3);
+            open = here && dsq <= v.rad2;
+            if (__any(here && !open)) {
+              soft = walk_soft_overlap(v, bg, rb, c3, dsq);
+              open = open || (here && soft && dsq <= v.rm2);
+            }
+          }
+          if (here) nd = v.link;
+          if (v.c0 < 0) {
+            if (open) {
+              if (FILL) a.parts[ppos + nruns] = {v.first, oid, v.count};
+              ++nruns;
+              nsrc += v.count;
+            }
+          } else if (open) {
             nd = v.c0;
           }
+          const bool cell = here && !open;
+          if (FILL && cell) {
+            const int at = soft ? spos + nsoft : hpos + nhex;
+            a.cells[at] = {cur, oid | b | (soft ? (int)0x80000000u : 0)};
+          }
+          nhex += cell && !soft;
+          nsoft += cell && soft;
+          const bool opens = open && v.c0 >= 0;
+          cur = __any(opens) ? v.c0 : v.link;
+          line.load(a.rec, max(cur, 0));
         }
       }
-  if (!FILL) {
+  if (!FILL && live) {
     a.nCell[b] = nhex + nsoft;
     a.nPart[b] = nruns;
     a.softStart[b] = nhex;
@@ -134,9 +186,10 @@ __global__ void walk_records_kernel(int nn, const double* node64, const int* fir
   const double r = g[3];
   double rad = kgeom * r / theta;
   if (rad < r) rad = r;
-  v.rad = rad;
+  v.rad2 = rad * rad;
   v.rs = 2.0 * g[4];
-  v.rm = kgeom * r / thetaMono;
+  const double rm = kgeom * r / thetaMono;
+  v.rm2 = rm * rm;
   v.count = count[nd];
   v.c0 = child[2 * nd];
   v.link = esc ? esc[nd] : child[2 * nd + 1];
@@ -280,6 +333,7 @@ static WalkWork work_layout(int nb, int nn, size_t scan) {
 static WalkArgs walk_args(const ChangaListBuild* L, int* err) {
   WalkArgs a;
   a.nb = L->nBuckets;
+  a.group = walk_group(a.nb);
   char* base = static_cast<char*>(L->work);
   a.nCell = reinterpret_cast<int*>(base + 256);
   a.nPart = a.nCell + (L->nBuckets + 1);
@@ -335,7 +389,7 @@ extern "C" int changaBuildListsCount(const ChangaListBuild* L, long long* numCel
                             const_cast<WalkRec*>(args.rec), s));
   }
   if (nb > 0) {
-    hipLaunchKernelGGL(walk_kernel<false>, dim3((nb + kWalkBlock - 1) / kWalkBlock),
+    hipLaunchKernelGGL(walk_kernel<false>, dim3((nb - 1) / args.group + 1),
                        dim3(kWalkBlock), 0, s, args);
     CGPU_CHECK(hipGetLastError());
   }
@@ -374,8 +428,9 @@ extern "C" int changaBuildListsFill(const ChangaListBuild* L, void* stream) {
     return fail("changaBuildListsFill: work buffer too small", hipErrorInvalidValue, __FILE__,
                 __LINE__);
   if (nb > 0) {
-    hipLaunchKernelGGL(walk_kernel<true>, dim3((nb + kWalkBlock - 1) / kWalkBlock),
-                       dim3(kWalkBlock), 0, s, walk_args(L, static_cast<int*>(L->work)));
+    const WalkArgs args = walk_args(L, static_cast<int*>(L->work));
+    hipLaunchKernelGGL(walk_kernel<true>, dim3((nb - 1) / args.group + 1), dim3(kWalkBlock), 0, s,
+                       args);
     CGPU_CHECK(hipGetLastError());
   }
   return 0;

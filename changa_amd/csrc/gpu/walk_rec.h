@@ -16,14 +16,14 @@
 
 namespace cgpu {
 
-// 64 bytes, one cache line per visited node: the centre of mass, the
-// opening radius, twice the softening, the monopole opening radius, the
-// particle count, the first child (c0 < 0: a bucket), a link and the first
+// 64 bytes, one cache line per visited node: the centre of mass, the square
+// of the opening radius, twice the softening, the square of the monopole
+// opening radius, the particle count, the first child (c0 < 0: a bucket), a link and the first
 // particle. The link is the second child for the cooperative walk and the
 // escape node (the depth-first successor of the node's subtree) for the
 // stackless depth-first walk of the list builder.
 struct alignas(16) WalkRec {
-  double cx, cy, cz, rad, rs, rm;
+  double cx, cy, cz, rad2, rs, rm2;
   int count, c0, link, first;
 };
 static_assert(sizeof(WalkRec) == 64, "one cache line per node");
@@ -37,19 +37,26 @@ hipError_t walk_records(int nn, const double* node64, const int* first, const in
 
 #pragma clang fp contract(off)
 
-__device__ __forceinline__ bool walk_box_sphere(const double* lo, const double* hi,
-                                                const double c[3], double r) {
+// squared distance of the point c from the box [lo, hi]
+__device__ __forceinline__ double walk_box_dsq(const double* lo, const double* hi,
+                                               const double c[3]) {
   double dsq = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    double e = 0.0;
-    if (c[k] < lo[k])
-      e = lo[k] - c[k];
-    else if (c[k] > hi[k])
-      e = c[k] - hi[k];
+    // lo - c below the box, c - hi above it, else 0 (lo <= hi): no branches
+    const double e = fmax(fmax(lo[k] - c[k], c[k] - hi[k]), 0.0);
     dsq += e * e;
   }
-  return dsq <= r * r;
+  return dsq;
+}
+
+// The softening of the node at c3, dsq from the bucket's box, overlaps the
+// bucket (bg, rb: see walk_decide).
+__device__ __forceinline__ bool walk_soft_overlap(const WalkRec& v, const double* bg, double rb,
+                                                  const double c3[3], double dsq) {
+  const double rs = v.rs;
+  const double dx = c3[0] - bg[0], dy = c3[1] - bg[1], dz = c3[2] - bg[2];
+  return dx * dx + dy * dy + dz * dz <= (rs + rb) * (rs + rb) || dsq <= rs * rs;
 }
 
 // 0 open, 1 hexadecapole cell, 2 softened cell. bg: the target bucket's
@@ -59,13 +66,10 @@ __device__ __forceinline__ int walk_decide(const WalkRec& v, const double* bg, d
                                            double oy, double oz) {
   if (v.count <= 6) return 0;
   const double c3[3] = {v.cx + ox, v.cy + oy, v.cz + oz};
-  if (walk_box_sphere(bg + 6, bg + 9, c3, v.rad)) return 0;
-  const double rs = v.rs;
-  const double dx = c3[0] - bg[0], dy = c3[1] - bg[1], dz = c3[2] - bg[2];
-  const bool soft_overlap = dx * dx + dy * dy + dz * dz <= (rs + rb) * (rs + rb) ||
-                            walk_box_sphere(bg + 6, bg + 9, c3, rs);
-  if (!soft_overlap) return 1;
-  return walk_box_sphere(bg + 6, bg + 9, c3, v.rm) ? 0 : 2;
+  const double dsq = walk_box_dsq(bg + 6, bg + 9, c3);
+  if (dsq <= v.rad2) return 0;
+  if (!walk_soft_overlap(v, bg, rb, c3, dsq)) return 1;
+  return dsq <= v.rm2 ? 0 : 2;
 }
 
 #pragma clang fp contract(on)
