@@ -31,8 +31,8 @@ int ltw_launch(const CudaMultipoleMoments* nodes, int numNodes, const CompactPar
                void* work, size_t workBytes, int maxCells, int maxRuns, int* errOut,
                hipStream_t s);
 // per-wavefront scratch of a local-tree-walk request: cells and particle runs
-// (229 KB a wavefront; a request runs at most one wavefront per 64
-// particles, up to the device's resident count)
+// (229 KB a wavefront; a request runs at most one wavefront per claim of
+// ltw.hip's 8 particles, up to the device's resident count)
 constexpr int kLtwMaxCells = 16384;
 constexpr int kLtwMaxRuns = 8192;
 #endif

@@ -54,6 +54,16 @@ constexpr int kLtwCounterStride = 32;
 constexpr int kLtwErrCapacity = 1;  // a walk exceeded maxCells / maxRuns or the stack
 constexpr int kLtwErrIndex = 2;     // a node or particle index outside its array
 
+// Particles a wavefront claims at a time: it takes the runs that start among
+// them. Few, because a run is a whole walk and its forces: with 64 a wavefront
+// did about six in sequence, a request ended with its slowest, and one of less
+// than 2^18 particles did not reach the resident wavefronts. us of a request
+// with 64 / 32 / 16 / 8 / 4: 4,096 particles 514 / 319 / 275 / 202 / 206,
+// 2^17 halos 860 / 611 / 568 / 523 / 528, 2^18 1,684 / 1,522 / 1,369 / 1,313 /
+// 1,331, 2^22 halos 12,820 / 12,213 / 11,992 / 11,917 / 12,239.
+constexpr int kLtwClaim = 8;
+static_assert(kLtwClaim <= kWave, "a lane looks at each");
+
 struct LtwArgs {
   ChangaGravityLaunch pc, pp;  // lists: the bases of the wavefronts' scratch
   const CudaMultipoleMoments* nodes;
@@ -271,8 +281,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void lt
   const int cbase = blockIdx.x * a.maxCells, rbase = blockIdx.x * a.maxRuns;
   ILCell* cells = a.cells + cbase;
   ILPart* runs = a.runs + rbase;
-  // chunks of 64 consecutive particles in kLtwRanges contiguous ranges
-  const int nchunk = (a.last - a.first) / kWave + 1;
+  // chunks of consecutive particles in kLtwRanges contiguous ranges
+  const int nchunk = (a.last - a.first) / kLtwClaim + 1;
   int q = blockIdx.x % kLtwRanges;
   for (int tried = 0; tried < kLtwRanges;) {
     const int r0 = (int)((long long)nchunk * q / kLtwRanges);
@@ -285,8 +295,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void lt
       q = q + 1 == kLtwRanges ? 0 : q + 1;
       continue;
     }
-    const int p0 = a.first + (r0 + k) * kWave;
-    const int np = min(kWave, a.last - p0 + 1);
+    const int p0 = a.first + (r0 + k) * kLtwClaim;
+    const int np = min(kLtwClaim, a.last - p0 + 1);
     // the runs (same nodeId) that start in this chunk
     const int nid = lane < np ? a.parts[p0 + lane].nodeId : -1;
     int prev = __shfl_up(nid, 1, kWave);
@@ -353,8 +363,8 @@ __global__ void ltw_reset_kernel(int* counters) {
   if (i < kLtwRanges * kLtwCounterStride + 1) counters[i] = 0;  // counters, then err
 }
 
-// Wavefronts of a request for n particles: the resident maximum, but no
-// more than its 64-particle chunks (each wavefront holds its own scratch).
+// Wavefronts of a request for n particles: the resident maximum, but no more
+// than its claims (each wavefront holds its own scratch).
 static int ltw_grid(int n, int* grid) {
   int dev = 0, ncu = 0, per = 0;
   CGPU_CHECK(hipGetDevice(&dev));
@@ -362,7 +372,7 @@ static int ltw_grid(int n, int* grid) {
   CGPU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)ltw_kernel, kWave,
                                                           0));
   const int full = ncu * (per > 0 ? per : 1);
-  const int nchunk = n > 0 ? (n - 1) / kWave + 1 : 1;
+  const int nchunk = n > 0 ? (n - 1) / kLtwClaim + 1 : 1;
   *grid = full < nchunk ? full : nchunk;
   return 0;
 }
