@@ -468,10 +468,14 @@ class Evaluation:
         b.parts = self.d_plist.data_ptr()
         gpu.check(gpu.lib().changaBuildListsFill(ctypes.byref(b), self._sp()),
                   "changaBuildListsFill")
-        cm = self.d_cmarks.cpu().numpy().astype(np.int64)
-        pm = self.d_pmarks.cpu().numpy().astype(np.int64)
-        ss = self.d_soft_start.cpu().numpy()[:nb].astype(np.int64)
-        src = d_src.cpu().numpy()[:nb].astype(np.int64)
+        # the marks are the count's, which has ended: on a stream of their own
+        # their downloads (each ends before it returns) and the sums below run
+        # beside the fill instead of after it
+        with torch.cuda.stream(torch.cuda.Stream(self.device)):
+            cm = self.d_cmarks.cpu().numpy().astype(np.int64)
+            pm = self.d_pmarks.cpu().numpy().astype(np.int64)
+            ss = self.d_soft_start.cpu().numpy()[:nb].astype(np.int64)
+            src = d_src.cpu().numpy()[:nb].astype(np.int64)
         self.t_lists = dict(cell_marks=cm, part_marks=pm, soft_start=ss)
         act = self.t_sizes.astype(np.int64)
         nhex, nsoft = ss - cm[:-1], cm[1:] - ss
