@@ -190,14 +190,16 @@ __global__ __launch_bounds__(kMomBlock) __attribute__((amdgpu_waves_per_eu(3))) 
     double lo0 = HUGE_VAL, lo1 = HUGE_VAL, lo2 = HUGE_VAL;
     double hi0 = -HUGE_VAL, hi1 = -HUGE_VAL, hi2 = -HUGE_VAL;
     double hm[kMomHeld], hx[kMomHeld], hy[kMomHeld], hz[kMomHeld], hs[kMomHeld];
+    if (cnt > 0) {  // (an empty leaf has no last particle to fall back on)
 #pragma unroll
-    for (int t = 0; t < kMomHeld; ++t) {
-      const int i = min(f + sub + 4 * t, f + cnt - 1);
-      hm[t] = mass[i];
-      hx[t] = pos[3 * (size_t)i];
-      hy[t] = pos[3 * (size_t)i + 1];
-      hz[t] = pos[3 * (size_t)i + 2];
-      hs[t] = soft[i];
+      for (int t = 0; t < kMomHeld; ++t) {
+        const int i = min(f + sub + 4 * t, f + cnt - 1);
+        hm[t] = mass[i];
+        hx[t] = pos[3 * (size_t)i];
+        hy[t] = pos[3 * (size_t)i + 1];
+        hz[t] = pos[3 * (size_t)i + 2];
+        hs[t] = soft[i];
+      }
     }
     auto first_pass = [&](double m, double x, double y, double z, double h) {
       M += m;
