@@ -30,9 +30,9 @@ int ltw_launch(const CudaMultipoleMoments* nodes, int numNodes, const CompactPar
                float thetaMono, int nReplicas, float fperiod, float fperiodY, float fperiodZ,
                void* work, size_t workBytes, int maxCells, int maxRuns, int* errOut,
                hipStream_t s);
-// per-wavefront scratch of a local-tree-walk request: cells and particle runs
-// (229 KB a wavefront; a request runs at most one wavefront per claim of
-// ltw.hip's 8 particles, up to the device's resident count)
+// full-size scratch slice of a local-tree-walk request: cells and particle
+// runs (229 KB; a request holds one per 64 particles, at most as many as the
+// device holds wavefronts, 940 MB, and 4 bytes a particle: ltw.hip)
 constexpr int kLtwMaxCells = 16384;
 constexpr int kLtwMaxRuns = 8192;
 #endif

@@ -39,6 +39,7 @@
 #error "ltw.hip belongs to the GPU_LOCAL_TREE_WALK build of the library"
 #endif
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -64,6 +65,16 @@ constexpr int kLtwErrIndex = 2;     // a node or particle index outside its arra
 constexpr int kLtwClaim = 8;
 static_assert(kLtwClaim <= kWave, "a lane looks at each");
 
+// A request holds scratch for one full-size slice (maxCells, maxRuns: 229 KB)
+// per 64 of its particles, up to the resident wavefronts. A request that does
+// not reach those gives each claim an eighth of a slice instead, and leaves
+// the runs whose lists do not fit there to a second launch, a wavefront per
+// full slice, over the same memory. (Lists of the timed shapes have at most
+// 887 cells and 145 particle runs; an eighth holds 2,048 and 1,024.) With a
+// full slice per claim a request of 2^15 particles held 940 MB for 117.
+constexpr int kLtwSliceParticles = 64;
+constexpr int kLtwShare = kLtwSliceParticles / kLtwClaim;  // claims' scratch per slice
+
 struct LtwArgs {
   ChangaGravityLaunch pc, pp;  // lists: the bases of the wavefronts' scratch
   const CudaMultipoleMoments* nodes;
@@ -74,8 +85,11 @@ struct LtwArgs {
   ILCell* cells;  // per wave: maxCells entries
   ILPart* runs;   // per wave: maxRuns entries
   int maxCells, maxRuns;
-  int* counters;  // kLtwRanges claim counters, kLtwCounterStride ints apart; then err
-  int* err;
+  int* counters;  // kLtwRanges claim counters, kLtwCounterStride ints apart; then err,
+  int* err;       // the number of runs left to the second launch and its claim counter
+  int* numLeft;
+  int* claimLeft;
+  int* left;  // their first particles; NULL: one launch of full slices
 };
 
 template <int PCT, int PPT>
@@ -190,11 +204,13 @@ __device__ __forceinline__ int ltw_decide(const LtwNode& v, const LtwBucket& b, 
 // Cooperative walk of one bucket (node bn) over the LDS stack: entries are
 // node indices (low kCoopNodeBits bits) with the replica code above. Cells
 // go to cells[0, nhex), softened cells to cells[maxCells - nsoft, maxCells),
-// particle runs to runs[0, nruns). Returns false (and raises err) when a
-// capacity or an index check fails.
+// particle runs to runs[0, nruns). Returns false when a capacity or an index
+// check fails: it raises err, or, where only the scratch is too small and
+// leave is not negative, leaves the run that begins at that particle to the
+// second launch.
 // ---------------------------------------------------------------------------
-__device__ bool ltw_walk(const LtwArgs& a, const LtwBucket& b, int lane, unsigned* stack,
-                         ILCell* cells, ILPart* runs, int& nhex, int& nsoft, int& nruns) {
+__device__ bool ltw_walk(const LtwArgs& a, const LtwBucket& b, int lane, int leave,
+                         unsigned* stack, ILCell* cells, ILPart* runs, int& nhex, int& nsoft, int& nruns) {
   nhex = nsoft = nruns = 0;
   const int R = a.R, W = 2 * R + 1, nrep = W * W * W;
   for (int k = lane; k < nrep; k += kWave) {
@@ -242,9 +258,12 @@ __device__ bool ltw_walk(const LtwArgs& a, const LtwBucket& b, int lane, unsigne
       __syncthreads();
       return false;
     }
-    if (nhex + ch + 2 * (nsoft + cs) > a.maxCells || nruns + cr > a.maxRuns ||
-        sp + cp > kCoopStack) {
-      if (lane == 0) atomicOr(a.err, kLtwErrCapacity);
+    const bool deep = sp + cp > kCoopStack;
+    if (nhex + ch + 2 * (nsoft + cs) > a.maxCells || nruns + cr > a.maxRuns || deep) {
+      if (lane == 0) {
+        if (leave >= 0 && !deep) a.left[atomicAdd(a.numLeft, 1)] = leave;
+        else atomicOr(a.err, kLtwErrCapacity);
+      }
       __syncthreads();
       return false;
     }
@@ -272,6 +291,8 @@ __device__ bool ltw_walk(const LtwArgs& a, const LtwBucket& b, int lane, unsigne
 // one to three targets per lane at three wavefronts (168 VGPRs) measured
 // 5-20% slower on the 2^22 halos, the 128^3 box and the 2^20 sphere (the
 // walk's load latency wants the fourth wavefront).
+// LEFT: the second launch, over the runs the first one left.
+template <bool LEFT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void ltw_kernel(
     LtwArgs a) {
   __shared__ float4 lds[LtwLds<kLtwPcTile, kLtwPpTile>::f4];
@@ -281,6 +302,69 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void lt
   const int cbase = blockIdx.x * a.maxCells, rbase = blockIdx.x * a.maxRuns;
   ILCell* cells = a.cells + cbase;
   ILPart* runs = a.runs + rbase;
+  // the run of particles of bucket node bn that starts at rs
+  auto run = [&](int rs, int bn) {
+    // its end: the first particle past it with another nodeId
+    int re = a.last + 1;
+    for (int q0 = rs + 1; q0 <= a.last; q0 += kWave) {
+      const int p = q0 + lane;
+      const unsigned long long m = __ballot(p <= a.last && a.parts[p].nodeId != bn);
+      if (m) {
+        re = q0 + __builtin_ctzll(m);
+        break;
+      }
+    }
+    if (bn < 0 || bn >= a.numNodes) {
+      if (lane == 0) atomicOr(a.err, kLtwErrIndex);
+      return;
+    }
+    LtwBucket b;
+    {
+      const CudaMultipoleMoments& m = a.nodes[bn];
+      b.cx = m.cm.x;
+      b.cy = m.cm.y;
+      b.cz = m.cm.z;
+      b.rb = 2.0f * m.soft;
+      b.lo[0] = m.lesser_corner.x;
+      b.lo[1] = m.lesser_corner.y;
+      b.lo[2] = m.lesser_corner.z;
+      b.hi[0] = m.greater_corner.x;
+      b.hi[1] = m.greater_corner.y;
+      b.hi[2] = m.greater_corner.z;
+    }
+    int nhex, nsoft, nruns;
+    const int leave = !LEFT && a.left ? rs : -1;
+    if (!ltw_walk(a, b, lane, leave, stack, cells, runs, nhex, nsoft, nruns)) return;
+    // softened cells (filled from the end of the region) moved behind the
+    // hexadecapole cells, so one cell loop covers both
+    if (nsoft > 0) {
+      for (int i = lane; i < nsoft; i += kWave) cells[nhex + i] = cells[a.maxCells - 1 - i];
+      __syncthreads();
+    }
+    for (int t0 = rs; t0 < re; t0 += kWave) {
+      const Lanes l = lanes_for<1>(lane, min(kWave, re - t0));
+      Target t[1];
+      load_targets<false, 1>(a.pc, t0, l, 0.0, 0.0, 0.0, t);
+      Acc64 acc[1] = {{0.0, 0.0, 0.0, 0.0, 0.0f}};
+      pc_cells<false, kLtwPcTile, false, 1, false>(a.pc, cbase, cbase + nhex + nsoft, 0.0, 0.0,
+                                                    0.0, t, l, lds, acc);
+      pp_sources<false, 1, kLtwPpTile, false, 1>(a.pp, rbase, rbase + nruns, 0.0, 0.0, 0.0, t, l,
+                                                 ps, acc);
+      reduce_store<1>(reinterpret_cast<char*>(lds), 0, {1, 0}, l, acc, a.pc.vars + t0);
+    }
+  };
+  if constexpr (LEFT) {
+    const int n = *a.numLeft;
+    // a wavefront's first one by its number: most requests leave none, and
+    // a claim each of 2,048 wavefronts took 15-20 us
+    for (int k = blockIdx.x; k < n;) {
+      const int rs = a.left[k];
+      run(rs, a.parts[rs].nodeId);
+      if (lane == 0) k = gridDim.x + atomicAdd(a.claimLeft, 1);
+      k = __builtin_amdgcn_readfirstlane(k);
+    }
+    return;
+  }
   // chunks of consecutive particles in kLtwRanges contiguous ranges
   const int nchunk = (a.last - a.first) / kLtwClaim + 1;
   int q = blockIdx.x % kLtwRanges;
@@ -305,105 +389,72 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void lt
     while (starts) {
       const int s = __builtin_ctzll(starts);
       starts &= starts - 1ull;
-      const int bn = __shfl(nid, s, kWave);
-      const int rs = p0 + s;
-      // the run's end: the first particle past it with another nodeId
-      int re = a.last + 1;
-      for (int q0 = rs + 1; q0 <= a.last; q0 += kWave) {
-        const int p = q0 + lane;
-        const unsigned long long m = __ballot(p <= a.last && a.parts[p].nodeId != bn);
-        if (m) {
-          re = q0 + __builtin_ctzll(m);
-          break;
-        }
-      }
-      if (bn < 0 || bn >= a.numNodes) {
-        if (lane == 0) atomicOr(a.err, kLtwErrIndex);
-        continue;
-      }
-      LtwBucket b;
-      {
-        const CudaMultipoleMoments& m = a.nodes[bn];
-        b.cx = m.cm.x;
-        b.cy = m.cm.y;
-        b.cz = m.cm.z;
-        b.rb = 2.0f * m.soft;
-        b.lo[0] = m.lesser_corner.x;
-        b.lo[1] = m.lesser_corner.y;
-        b.lo[2] = m.lesser_corner.z;
-        b.hi[0] = m.greater_corner.x;
-        b.hi[1] = m.greater_corner.y;
-        b.hi[2] = m.greater_corner.z;
-      }
-      int nhex, nsoft, nruns;
-      if (!ltw_walk(a, b, lane, stack, cells, runs, nhex, nsoft, nruns)) continue;
-      // softened cells (filled from the end of the region) moved behind the
-      // hexadecapole cells, so one cell loop covers both
-      if (nsoft > 0) {
-        for (int i = lane; i < nsoft; i += kWave) cells[nhex + i] = cells[a.maxCells - 1 - i];
-        __syncthreads();
-      }
-      for (int t0 = rs; t0 < re; t0 += kWave) {
-        const Lanes l = lanes_for<1>(lane, min(kWave, re - t0));
-        Target t[1];
-        load_targets<false, 1>(a.pc, t0, l, 0.0, 0.0, 0.0, t);
-        Acc64 acc[1] = {{0.0, 0.0, 0.0, 0.0, 0.0f}};
-        pc_cells<false, kLtwPcTile, false, 1, false>(a.pc, cbase, cbase + nhex + nsoft, 0.0,
-                                                      0.0, 0.0, t, l, lds, acc);
-        pp_sources<false, 1, kLtwPpTile, false, 1>(a.pp, rbase, rbase + nruns, 0.0, 0.0, 0.0, t,
-                                                   l, ps, acc);
-        reduce_store<1>(reinterpret_cast<char*>(lds), 0, {1, 0}, l, acc, a.pc.vars + t0);
-      }
+      run(p0 + s, __shfl(nid, s, kWave));
     }
   }
 }
 
+constexpr int kLtwHead = kLtwRanges * kLtwCounterStride + 3;  // counters, err, numLeft, claimLeft
+
 __global__ void ltw_reset_kernel(int* counters) {
   const int i = threadIdx.x;
-  if (i < kLtwRanges * kLtwCounterStride + 1) counters[i] = 0;  // counters, then err
+  if (i < kLtwHead) counters[i] = 0;
 }
 
-// Wavefronts of a request for n particles: the resident maximum, but no more
-// than its claims (each wavefront holds its own scratch).
-static int ltw_grid(int n, int* grid) {
+// How a request for n particles runs: `slices` full-size scratch slices; with
+// share == 1 a wavefront per slice, else `waves` wavefronts of 1 / share of a
+// slice each and a second launch over the runs that they leave.
+struct LtwPlan {
+  int slices, waves, share;
+};
+
+static int ltw_plan(int n, LtwPlan* plan) {
   int dev = 0, ncu = 0, per = 0;
   CGPU_CHECK(hipGetDevice(&dev));
   CGPU_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  CGPU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)ltw_kernel, kWave,
-                                                          0));
+  CGPU_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)ltw_kernel<false>,
+                                                          kWave, 0));
   const int full = ncu * (per > 0 ? per : 1);
-  const int nchunk = n > 0 ? (n - 1) / kLtwClaim + 1 : 1;
-  *grid = full < nchunk ? full : nchunk;
+  auto pieces = [&](int particles) { return n > 0 ? (n - 1) / particles + 1 : 1; };
+  plan->slices = pieces(kLtwSliceParticles);
+  plan->share = kLtwShare;
+  if (plan->slices >= full) {
+    plan->slices = full;
+    plan->share = 1;
+  }
+  plan->waves = plan->share == 1 ? full : std::min(full, pieces(kLtwClaim));
   return 0;
 }
 
-// work buffer: claim counters and error flag (256-byte aligned head), then
-// the per-wavefront cell and run scratch
+// work buffer: claim counters and flags (256-byte aligned head), the slices'
+// cells, their particle runs, then the list of runs left
 struct LtwWork {
-  size_t cells, runs, total;
+  size_t cells, runs, left, total;
 };
 
-static LtwWork ltw_layout(int grid, int maxCells, int maxRuns) {
+static LtwWork ltw_layout(int n, const LtwPlan& p, int maxCells, int maxRuns) {
+  auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
   LtwWork w;
-  w.cells = 256 * ((sizeof(int) * (kLtwRanges * kLtwCounterStride + 1) + 255) / 256);
-  w.runs = w.cells + 256 * (((size_t)grid * maxCells * sizeof(ILCell) + 255) / 256);
-  w.total = w.runs + (size_t)grid * maxRuns * sizeof(ILPart);
+  w.cells = align(sizeof(int) * kLtwHead);
+  w.runs = w.cells + align((size_t)p.slices * maxCells * sizeof(ILCell));
+  w.left = w.runs + (size_t)p.slices * maxRuns * sizeof(ILPart);
+  w.total = w.left + (p.share > 1 ? sizeof(int) * (size_t)n : 0);
   return w;
 }
 
 // Work bytes of a request for n particles.
 int ltw_work_bytes(int n, int maxCells, int maxRuns, size_t* bytes) {
-  int grid = 0;
-  if (int e = ltw_grid(n, &grid)) return e;
-  if ((long long)grid * maxCells > 0x7fffffffll || (long long)grid * maxRuns > 0x7fffffffll)
+  LtwPlan p;
+  if (int e = ltw_plan(n, &p)) return e;
+  if ((long long)p.slices * maxCells > 0x7fffffffll || (long long)p.slices * maxRuns > 0x7fffffffll)
     return fail("local tree walk: scratch capacities exceed the int32 index range",
                 hipErrorInvalidValue, __FILE__, __LINE__);
-  *bytes = ltw_layout(grid, maxCells, maxRuns).total;
+  *bytes = ltw_layout(n, p, maxCells, maxRuns).total;
   return 0;
 }
 
 // One local-tree-walk request: the checks of the arguments, the counter
-// reset, the walk-and-force launch and the copy of its error flag to errOut
+// reset, the walk-and-force launches and the copy of their error flag to errOut
 // (device or pinned host memory).
 int ltw_launch(const CudaMultipoleMoments* nodes, int numNodes, const CompactPartData* parts,
                int numParts, VariablePartData* vars, int first, int last, int root, float theta,
@@ -424,14 +475,14 @@ int ltw_launch(const CudaMultipoleMoments* nodes, int numNodes, const CompactPar
     return fail("local tree walk: periodic replicas need fperiod, fperiodY, fperiodZ > 0",
                 hipErrorInvalidValue, __FILE__, __LINE__);
   const int n = last - first + 1;
-  int grid = 0;
-  if (int e = ltw_grid(n, &grid)) return e;
+  LtwPlan plan;
+  if (int e = ltw_plan(n, &plan)) return e;
   size_t need = 0;
   if (int e = ltw_work_bytes(n, maxCells, maxRuns, &need)) return e;
   if (workBytes < need)
     return fail("local tree walk: work buffer too small", hipErrorInvalidValue, __FILE__,
                 __LINE__);
-  const LtwWork L = ltw_layout(grid, maxCells, maxRuns);
+  const LtwWork L = ltw_layout(n, plan, maxCells, maxRuns);
   char* wb = static_cast<char*>(work);
   LtwArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -462,15 +513,25 @@ int ltw_launch(const CudaMultipoleMoments* nodes, int numNodes, const CompactPar
   a.err = a.counters + kLtwRanges * kLtwCounterStride;
   a.cells = reinterpret_cast<ILCell*>(wb + L.cells);
   a.runs = reinterpret_cast<ILPart*>(wb + L.runs);
-  a.maxCells = maxCells;
-  a.maxRuns = maxRuns;
+  a.numLeft = a.err + 1;
+  a.claimLeft = a.err + 2;
+  // (waves x the shares fit the slices: waves <= share x slices)
+  a.maxCells = maxCells / plan.share;
+  a.maxRuns = maxRuns / plan.share;
+  a.left = plan.share > 1 ? reinterpret_cast<int*>(wb + L.left) : nullptr;
   a.pc.list = a.cells;
   a.pp.list = a.runs;
-  hipLaunchKernelGGL(ltw_reset_kernel, dim3(1), dim3(kLtwRanges * kLtwCounterStride + 1), 0, s,
-                     a.counters);
+  hipLaunchKernelGGL(ltw_reset_kernel, dim3(1), dim3(kLtwHead), 0, s, a.counters);
   CGPU_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(ltw_kernel, dim3(grid), dim3(kWave), 0, s, a);
+  hipLaunchKernelGGL(ltw_kernel<false>, dim3(plan.waves), dim3(kWave), 0, s, a);
   CGPU_CHECK(hipGetLastError());
+  if (plan.share > 1) {
+    LtwArgs b = a;
+    b.maxCells = maxCells;
+    b.maxRuns = maxRuns;
+    hipLaunchKernelGGL(ltw_kernel<true>, dim3(plan.slices), dim3(kWave), 0, s, b);
+    CGPU_CHECK(hipGetLastError());
+  }
   if (errOut) CGPU_CHECK(hipMemcpyAsync(errOut, a.err, sizeof(int), hipMemcpyDefault, s));
   return 0;
 }
