@@ -139,6 +139,19 @@ __device__ __forceinline__ void radial32_fast(float r2, float hole, float alpha,
   }
 }
 
+// LDS beside the k-space table, whose size is the caller's: 32 bytes an entry,
+// in all at most the CU's 160 KB (4,348 entries). The runtime does not refuse
+// a launch that asks for more, the queue aborts; launch_ewald checks.
+struct EwLds {
+  // lattice offsets (n L, hole flag): all of them, then those that some
+  // particle of the wavefront needs, in place
+  float4 cand[kEwBlock / kWave][kEwMaxCand];
+  // the k-space table as weights on the cube |h_i| <= kEwCube (zero off the table)
+  float2 cube[kEwCubeN];
+  int n_outside, n_uneven;
+};
+constexpr size_t kEwLdsMax = 160 * 1024;
+
 __global__ __launch_bounds__(kEwBlock) __attribute__((amdgpu_waves_per_eu(5))) void ewald_kernel(const CompactPartData* parts,
                                                          VariablePartData* vars,
                                                          const int* markers, int first, int n,
@@ -146,13 +159,10 @@ __global__ __launch_bounds__(kEwBlock) __attribute__((amdgpu_waves_per_eu(5))) v
                                                          const double* root, EwaldParams p) {
   // h-loop table: per entry (k, hC) and (h as integers, hS); dynamic size
   extern __shared__ float4 sh[];
-  // lattice offsets (n L, hole flag) that some particle of the wavefront needs
-  __shared__ float4 cand[kEwBlock / kWave][kEwMaxCand];
-  __shared__ int lattice[kEwMaxCand];
-
-  // the same table as weights on the cube |h_i| <= kEwCube (zero off the table)
-  __shared__ float2 cube[kEwCubeN];
-  __shared__ int n_outside, n_uneven;
+  __shared__ EwLds lds;
+  auto& cand = lds.cand;
+  auto& cube = lds.cube;
+  int &n_outside = lds.n_outside, &n_uneven = lds.n_uneven;
 
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
   const float kscale = (float)(p.L / (2.0 * M_PI));  // k -> integer h
@@ -217,23 +227,25 @@ __global__ __launch_bounds__(kEwBlock) __attribute__((amdgpu_waves_per_eu(5))) v
       lo[k] = fminf(lo[k], __shfl_xor(lo[k], m, kWave));
       hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], m, kWave));
     }
-  // the lattice vectors, found once for the block: n + 3 in bytes, bit 24 hole
+  // the lattice vectors, found once for the block
   const int W = 2 * p.nEwReps + 1, NC = W * W * W;
+  const float Lf = (float)p.L, cut2f = (float)p.cut2;
   for (int c = tid; c < NC; c += kEwBlock) {
     const int ix = c / (W * W) - p.nEwReps, iy = (c / W) % W - p.nEwReps, iz = c % W - p.nEwReps;
     const bool hole = abs(ix) <= p.nReps && abs(iy) <= p.nReps && abs(iz) <= p.nReps;
-    lattice[c] = (ix + 3) | ((iy + 3) << 8) | ((iz + 3) << 16) | ((int)hole << 24);
+#pragma unroll
+    for (int w = 0; w < kEwBlock / kWave; ++w)
+      cand[w][c] = make_float4(ix * Lf, iy * Lf, iz * Lf, hole ? 1.0f : 0.0f);
   }
-  const float Lf = (float)p.L, cut2f = (float)p.cut2;
   __syncthreads();
-  // those that some particle of the wavefront needs, compacted
+  // those that some particle of the wavefront needs, compacted: a step writes
+  // at most as many entries as were read up to its end, after its reads
   int nc = 0;
   for (int c0 = 0; c0 < NC; c0 += kWave) {
     const int c = c0 + lane;
-    const int v = lattice[min(c, NC - 1)];
-    const float n[3] = {(float)((v & 255) - 3) * Lf, (float)(((v >> 8) & 255) - 3) * Lf,
-                        (float)(((v >> 16) & 255) - 3) * Lf};
-    const bool hole = (v >> 24) != 0, centre = (v & 0xffffff) == 0x030303;
+    const float4 v = cand[wv][min(c, NC - 1)];
+    const float n[3] = {v.x, v.y, v.z};
+    const bool hole = v.w != 0.0f, centre = v.x == 0.0f && v.y == 0.0f && v.z == 0.0f;
     float d2 = 0.f;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -244,9 +256,7 @@ __global__ __launch_bounds__(kEwBlock) __attribute__((amdgpu_waves_per_eu(5))) v
     // slack for FP32 rounding of the bound; the per-particle test is exact
     const bool need = c < NC && !centre && (hole || d2 <= cut2f * 1.0001f + 1e-6f * Lf * Lf);
     const unsigned long long mask = __ballot(need);
-    if (need)
-      cand[wv][nc + __popcll(mask & ((1ull << lane) - 1ull))] =
-          make_float4(n[0], n[1], n[2], hole ? 1.0f : 0.0f);
+    if (need) cand[wv][nc + __popcll(mask & ((1ull << lane) - 1ull))] = v;
     nc += __popcll(mask);
   }
   __syncthreads();
@@ -371,6 +381,9 @@ int launch_ewald(const CompactPartData* parts, VariablePartData* vars, const int
   if (p.nEwReps > 3)
     return fail("Ewald: nEwReps > 3", hipErrorInvalidValue, __FILE__, __LINE__);
   size_t shm = sizeof(float4) * 2 * (size_t)(p.nH > 0 ? p.nH : 1);
+  if (sizeof(EwLds) + shm > kEwLdsMax)
+    return fail("Ewald: nEwhLoop too large (its table is staged in LDS)", hipErrorInvalidValue,
+                __FILE__, __LINE__);
   int blocks = (n + kEwBlock - 1) / kEwBlock;
   hipLaunchKernelGGL(ewald_kernel, dim3(blocks), dim3(kEwBlock), shm, s, parts, vars, markers,
                      first, n, d_ewt, pos64, d_root, p);
