@@ -59,16 +59,22 @@ pc_kernel(ChangaGravityLaunch a) {
 }
 
 // ---------------------------------------------------------------------------
-// Per-bucket particle-particle kernel (KIND: see pp_sources).
+// Per-bucket particle-particle kernel (KIND: see pp_sources). TEAM: the build
+// for several wavefronts per bucket. The one for a single wavefront has its
+// tiles in a static array and no team arithmetic: 2^20 sphere 404 us against
+// 419 for the TEAM build with one wavefront, 128^3 box 596 / 612, 2^22 halos
+// 2,872 / 2,905 (half of it from the array: its LDS addresses are constants).
 // ---------------------------------------------------------------------------
-template <bool PRECISE, int KIND>
-__global__ __launch_bounds__(kWave * kTeamWaves) __attribute__((amdgpu_waves_per_eu(4))) void
-pp_kernel(ChangaGravityLaunch a) {
+template <bool PRECISE, int KIND, bool TEAM>
+__global__ __launch_bounds__(kWave * (TEAM ? kTeamWaves : 1))
+__attribute__((amdgpu_waves_per_eu(4))) void pp_kernel(ChangaGravityLaunch a) {
   // staged tiles of each wavefront; reused for the slot reduction at the end
   // of each chunk
-  extern __shared__ float4 lds[];
+  extern __shared__ float4 team_lds[];
+  __shared__ float4 own_lds[TEAM ? 1 : kPpLds];
+  float4* lds = TEAM ? team_lds : own_lds;
   const int lane = threadIdx.x & (kWave - 1);
-  const Team team = block_team();
+  const Team team = TEAM ? block_team() : Team{1, 0};
   PpFwdLds<kPpTile>& s = *reinterpret_cast<PpFwdLds<kPpTile>*>(lds + team.wave * kPpLds);
 
   const int b = xcd_bucket(blockIdx.x, a.numBuckets);
@@ -94,6 +100,13 @@ pp_kernel(ChangaGravityLaunch a) {
                       a.vars + bstart + t0);
     });
   }
+}
+
+template <bool TEAM>
+static auto pick_pp(const ChangaGravityLaunch& a) {
+  if (a.listKind == 0)
+    return a.tpos64 ? pp_kernel<true, 0, TEAM> : pp_kernel<false, 0, TEAM>;
+  return a.tpos64 ? pp_kernel<true, 1, TEAM> : pp_kernel<false, 1, TEAM>;
 }
 
 // 128-byte cell records (kCellRecFloats): centre of mass as 3 doubles, mass,
@@ -225,11 +238,9 @@ extern "C" int changaPartGravity(const ChangaGravityLaunch* a, void* stream) {
   // with 1 / 2 / 4 wavefronts per bucket, 2,074 25 / 23 / 25, 3,850 16 / 19 /
   // 30, 7,985 43 / 52 / 72
   const int waves = team_waves(a->numBuckets, 1024, 2048);
-  const bool pr = a->tpos64 != nullptr;
-  const auto kernel = a->listKind == 0 ? (pr ? pp_kernel<true, 0> : pp_kernel<false, 0>)
-                                       : (pr ? pp_kernel<true, 1> : pp_kernel<false, 1>);
+  const auto kernel = waves > 1 ? pick_pp<true>(*a) : pick_pp<false>(*a);
   hipLaunchKernelGGL(kernel, dim3(a->numBuckets), dim3(kWave * waves),
-                     waves * kPpLds * sizeof(float4), s, *a);
+                     waves > 1 ? waves * kPpLds * sizeof(float4) : 0, s, *a);
   CGPU_CHECK(hipGetLastError());
   return 0;
 }
