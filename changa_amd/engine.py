@@ -462,20 +462,24 @@ class Evaluation:
         gpu.check(gpu.lib().changaBuildListsCount(ctypes.byref(b), ctypes.byref(nc),
                                                   ctypes.byref(npr), self._sp()),
                   "changaBuildListsCount")
+        # the marks are the count's: their copies go ahead of the fill, and the
+        # sums below run beside it
+        marks = (self.d_cmarks, self.d_pmarks, self.d_soft_start[:nb], d_src[:nb])
+        host_marks = torch.empty(sum(len(t) for t in marks), dtype=torch.int32, pin_memory=True)
+        with torch.cuda.stream(self.stream):
+            for dst, src in zip(host_marks.split([len(t) for t in marks]), marks):
+                dst.copy_(src, non_blocking=True)
+            copied = torch.cuda.Event()
+            copied.record()
         self.d_cells = torch.empty((max(nc.value, 1), 2), **i32)
         self.d_plist = torch.empty((max(npr.value, 1), 3), **i32)
         b.cells = self.d_cells.data_ptr()
         b.parts = self.d_plist.data_ptr()
         gpu.check(gpu.lib().changaBuildListsFill(ctypes.byref(b), self._sp()),
                   "changaBuildListsFill")
-        # the marks are the count's, which has ended: on a stream of their own
-        # their downloads (each ends before it returns) and the sums below run
-        # beside the fill instead of after it
-        with torch.cuda.stream(torch.cuda.Stream(self.device)):
-            cm = self.d_cmarks.cpu().numpy().astype(np.int64)
-            pm = self.d_pmarks.cpu().numpy().astype(np.int64)
-            ss = self.d_soft_start.cpu().numpy()[:nb].astype(np.int64)
-            src = d_src.cpu().numpy()[:nb].astype(np.int64)
+        copied.synchronize()
+        cm, pm, ss, src = np.split(host_marks.numpy().astype(np.int64),
+                                   np.cumsum([len(t) for t in marks])[:-1])
         self.t_lists = dict(cell_marks=cm, part_marks=pm, soft_start=ss)
         act = self.t_sizes.astype(np.int64)
         nhex, nsoft = ss - cm[:-1], cm[1:] - ss
