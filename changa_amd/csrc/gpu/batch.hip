@@ -228,8 +228,14 @@ namespace {
 // Wavefronts per bucket of the persistent kernel. us with 1 / 2 / 4 (medians
 // over the tuned configurations): 541 buckets 88 / 50 / 34, 2,074 90 / 64 / 59,
 // 4,051 114 / 94 / 95, 7,985 174 / 161 / 172, 12,004 603 / 599 / 642, 15,948
-// 314 / 309 / 341, 20,185 of a sparse rung 188 / 199 / 265.
-int batch_waves(int buckets) { return team_waves(buckets, 2048, 8192); }
+// 314 / 309 / 341, 20,185 of a sparse rung 188 / 199 / 265. The launch is made
+// to have the card to itself. Where it has not, teams cost: 8 plans on 8
+// streams, 1,203 / 1,550 / 1,872 buckets, 305 / 382 / 454 us with four, 229 /
+// 310 / 380 with two, 217 / 268 / 310 with one (a single one 61 / 71 / 77, 59 /
+// 71 / 80, 78 / 86 / 92), so four stop at 1,024, where two are as good; 6,049
+// buckets 1,177 with two and 1,076 with one, where a single one takes 180 and
+// 199, so two stay.
+int batch_waves(int buckets) { return team_waves(buckets, 1024, 8192); }
 
 // Workgroups of the persistent kernel over this many buckets: those resident
 // on the whole device, but no more than there are buckets to claim. -1 on error.

@@ -198,8 +198,12 @@ extern "C" int changaNodeGravity(const ChangaGravityLaunch* a, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   // us with 1 / 2 / 4 wavefronts per bucket: 541 buckets 18 / 12 / 11, 2,074
   // 41 / 34 / 32, 7,985 136 / 129 / 136, 15,948 262 / 263 / 278, 20,185 of a
-  // sparse rung 109 / 129 / 178
-  const int waves = team_waves(a->numBuckets, 2048, 8192);
+  // sparse rung 109 / 129 / 178. Four stop at 1,024 because requests also come
+  // on several streams, which fill the card by themselves: cells and particles
+  // of 8 requests on 8 streams took 264 / 333 us at 1,550 / 1,872 buckets with
+  // four, 231 / 304 with two, 220 / 275 with one (a single one 57 / 66, 61 /
+  // 66, 74 / 80).
+  const int waves = team_waves(a->numBuckets, 1024, 8192);
   const auto kernel = a->cellRecords ? (a->tpos64 ? pc_kernel<true, true> : pc_kernel<false, true>)
                                      : (a->tpos64 ? pc_kernel<true, false> : pc_kernel<false, false>);
   hipLaunchKernelGGL(kernel, dim3(a->numBuckets), dim3(kWave * waves),
@@ -236,7 +240,9 @@ extern "C" int changaPartGravity(const ChangaGravityLaunch* a, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   // the lists are a third of the cells' in time: 541 buckets 23 / 17 / 13 us
   // with 1 / 2 / 4 wavefronts per bucket, 2,074 25 / 23 / 25, 3,850 16 / 19 /
-  // 30, 7,985 43 / 52 / 72
+  // 30, 7,985 43 / 52 / 72. (Two of 1,550 / 1,872 buckets: 26 / 29 us against
+  // 34 / 36 with one; 8 streams of them 108 / 128 against 95 / 104, which the
+  // cells' kernels more than make up.)
   const int waves = team_waves(a->numBuckets, 1024, 2048);
   const auto kernel = waves > 1 ? pick_pp<true>(*a) : pick_pp<false>(*a);
   hipLaunchKernelGGL(kernel, dim3(a->numBuckets), dim3(kWave * waves),
