@@ -52,15 +52,15 @@ template <int PCT, int PPT>
 struct BatchLds {
   static constexpr size_t pc = (size_t)(PCT + 1) * kFwdRec * sizeof(float);
   static constexpr size_t pp = sizeof(PpFwdLds<PPT>);
-  static constexpr size_t red = reduce_bytes<3>();
+  static constexpr size_t red = reduce_bytes<2>();
   static constexpr size_t bytes = pc > pp ? (pc > red ? pc : red) : (pp > red ? pp : red);
   static constexpr size_t f4 = (bytes + 15) / 16;
 };
 
 // One bucket: cells, then particles, then one update of its results. Every
 // phase that uses LDS ends with a barrier, so the phases share one buffer.
-// KMAX 1: one target per lane; 3: one to three, chosen per chunk by its size
-// (targets_per_lane). REC: cells from the 128-byte cell records.
+// KMAX, the plan's targetsPerLane: 1: one; 3: one or two, chosen per chunk by
+// its size (targets_per_lane). REC: cells from the 128-byte cell records.
 template <bool PRECISE, int KIND, int PCT, int PPT, int KMAX, bool REC>
 __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane, const Team& team,
                                              float4* lds_all) {
@@ -90,7 +90,7 @@ __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane
                       a.pc.vars + bstart + t0);
     };
     if constexpr (KMAX == 1) chunk(KTag<1>());
-    else with_targets_per_lane(nt, chunk);
+    else with_targets_per_lane<2, true>(nt, chunk);
   }
 }
 
@@ -101,11 +101,11 @@ __device__ __forceinline__ void batch_bucket(const BatchArgs& a, int b, int lane
 // wavefronts of a workgroup see the same claim.
 // Four wavefronts per SIMD (128 VGPRs), because the FP32 VALU issues the
 // force loops faster with four than with three (gravity_body.h: pc_cells).
-// KMAX 1 holds one chunk loop and does not spill: on a sparse rung (one to
-// three targets in most buckets), where a tile's own work weighs most, it
-// measured 7.69 ms against 11.6 for KMAX 3, whose three-targets loop spills
-// 28 to 42 registers around the tiles; on the dense 2^22 halos, where the
-// shared LDS reads weigh more, KMAX 3 measured 9.13 ms against 9.92.
+// No third target per lane: its loop spills 28 to 50 registers, which every
+// bucket pays for. Records, ms with up to three and with up to two: 2^18
+// sphere in buckets of 4 / 8 / 16 / 32 targets 1.24 / .80 / .63 / .67 and .91
+// / .66 / .58 / .66, 128^3 box 2.79 and 2.49, 2^22 halos 9.77 and 9.23. KMAX 1
+// holds one chunk loop.
 template <bool PRECISE, int KIND, int PCT, int PPT, int KMAX, bool REC>
 __global__ __launch_bounds__(kWave * kTeamWaves) __attribute__((amdgpu_waves_per_eu(4))) void
 batch_kernel(BatchArgs a) {
@@ -459,7 +459,7 @@ extern "C" int changaBatchPlanCreate(const ChangaGravityLaunch* cells,
     };
     // Every candidate is timed over 2 runs; the 4 fastest and the default
     // configuration (cell tile 64, particle tile 256, one bucket per claim,
-    // tree order, up to three targets per lane, wire moments) are timed again
+    // tree order, several targets per lane, wire moments) are timed again
     // over 6 runs, and the default is kept unless another is more than 2%
     // faster, so that variants of near-equal time do not flip from one plan
     // to the next. The default runs twice, untimed, before the sweep.

@@ -41,7 +41,7 @@ pc_kernel(ChangaGravityLaunch a) {
 
   for (int t0 = 0; t0 < n; t0 += kWave) {
     const int nt = min(kWave, n - t0);
-    with_targets_per_lane<2>(nt, [&](auto kt) {
+    with_targets_per_lane<2, true>(nt, [&](auto kt) {
       constexpr int K = decltype(kt)::value;
       const Lanes l = lanes_for<K>(lane, nt);
       Target t[K];

@@ -445,15 +445,14 @@ __device__ __forceinline__ Lanes lanes_for(int lane, int nt) {
 // nslot(K) nt / (64 K). CELLS (the chunk runs a cell loop): the larger K on
 // ties, because every lane of a slot reads a staged cell's whole record and K
 // targets share those eight LDS reads (16 targets: 348 cycles per wavefront
-// evaluation with K = 2, 379 with K = 1), and at most two up to 16 targets
-// (K = 3 only adds places there, and the batched kernel spills for it: 128^3
-// box 2.54 ms, 2.50 with K <= 2). Particles alone (one LDS read per source):
-// the smaller K on ties (128^3 box 0.60 ms, 0.63 with the larger).
-template <int LIM = 3, bool CELLS = true>
+// evaluation with K = 2, 379 with K = 1), and at most two (three spill at
+// four wavefronts per SIMD: batch.hip). Particles alone (one LDS read per
+// source): the smaller K on ties (128^3 box 0.60 ms, 0.63 with the larger).
+template <int LIM, bool CELLS>
 __device__ __forceinline__ int targets_per_lane(int nt) {
   int best = 1;
   int bnum = (kWave / nt) * nt, bden = 1;  // utilisation bnum / (64 bden)
-  for (int k = 2; k <= (CELLS && nt <= 16 ? 2 : LIM); ++k) {
+  for (int k = 2; k <= LIM; ++k) {
     const int ng = (nt + k - 1) / k;
     const int num = (kWave / ng) * nt;
     if (num * bden + (CELLS ? 1 : 0) > bnum * k) {
@@ -472,9 +471,9 @@ struct KTag {
 
 // Calls body(KTag<K>()) with K = targets_per_lane(nt) (nt uniform across the
 // wavefront, so one of the instantiations runs).
-template <int LIM = 3, bool CELLS = true, typename Body>
+template <int LIM, bool CELLS, typename Body>
 __device__ __forceinline__ void with_targets_per_lane(int nt, Body&& body) {
-  static_assert(LIM == 2 || LIM == 3, "targets per lane");
+  static_assert(LIM == 2 || (LIM == 3 && !CELLS), "targets per lane");
   const int k = targets_per_lane<LIM, CELLS>(nt);
   if (k == 1) {
     body(KTag<1>());
