@@ -433,10 +433,10 @@ class Evaluation:
         nb = len(keep)
         i32 = dict(dtype=torch.int32, device=self.device)
         self.d_bucket_node = self._bucket_nodes()
-        self.d_cmarks = torch.empty(nb + 1, **i32)
-        self.d_pmarks = torch.empty(nb + 1, **i32)
-        self.d_soft_start = torch.empty(max(nb, 1), **i32)
-        d_src = torch.empty(max(nb, 1), **i32)
+        # one array, so that one copy brings all to the host; rows whole lines apart
+        marks = torch.empty((4, (nb + 32) // 32 * 32), **i32)
+        self.d_cmarks, self.d_pmarks = marks[0, :nb + 1], marks[1, :nb + 1]
+        self.d_soft_start, d_src = marks[2], marks[3]
         nbytes = gpu.lib().changaBuildListsWorkBytes(nb, tr["n_nodes"])
         if nbytes == 0:
             raise RuntimeError("changaBuildListsWorkBytes failed")
@@ -462,13 +462,14 @@ class Evaluation:
         gpu.check(gpu.lib().changaBuildListsCount(ctypes.byref(b), ctypes.byref(nc),
                                                   ctypes.byref(npr), self._sp()),
                   "changaBuildListsCount")
-        # the marks are the count's: their copies go ahead of the fill, and the
-        # sums below run beside it
-        marks = (self.d_cmarks, self.d_pmarks, self.d_soft_start[:nb], d_src[:nb])
-        host_marks = torch.empty(sum(len(t) for t in marks), dtype=torch.int32, pin_memory=True)
+        # the marks are the count's: their one copy goes ahead of the fill, and
+        # the sums below run beside it (on a stream of its own the copy would
+        # cost less, but with one stream more a caller's streams share the four
+        # hardware queues: cell and particle kernels of four evaluations on
+        # four streams took 37% longer)
+        host_marks = torch.empty(marks.shape, dtype=torch.int32, pin_memory=True)
         with torch.cuda.stream(self.stream):
-            for dst, src in zip(host_marks.split([len(t) for t in marks]), marks):
-                dst.copy_(src, non_blocking=True)
+            host_marks.copy_(marks, non_blocking=True)
             copied = torch.cuda.Event()
             copied.record()
         self.d_cells = torch.empty((max(nc.value, 1), 2), **i32)
@@ -478,8 +479,9 @@ class Evaluation:
         gpu.check(gpu.lib().changaBuildListsFill(ctypes.byref(b), self._sp()),
                   "changaBuildListsFill")
         copied.synchronize()
-        cm, pm, ss, src = np.split(host_marks.numpy().astype(np.int64),
-                                   np.cumsum([len(t) for t in marks])[:-1])
+        h = host_marks.numpy()
+        cm, pm = h[0, :nb + 1].astype(np.int64), h[1, :nb + 1].astype(np.int64)
+        ss, src = h[2, :nb].astype(np.int64), h[3, :nb].astype(np.int64)
         self.t_lists = dict(cell_marks=cm, part_marks=pm, soft_start=ss)
         act = self.t_sizes.astype(np.int64)
         nhex, nsoft = ss - cm[:-1], cm[1:] - ss
