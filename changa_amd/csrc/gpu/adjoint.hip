@@ -217,12 +217,6 @@ __device__ __forceinline__ void spline_bc(float r2, float twoh, float& b, float&
   }
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = kWave / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
-  return v;
-}
-
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -282,7 +276,6 @@ struct AdjArgs {
   Transpose tr;
   PartTranspose ptr;
   int nNodes;
-  int entries;
 };
 
 // ---------------------------------------------------------------------------
@@ -333,7 +326,7 @@ __global__ void adj_item_heads_kernel(const int* item, const int* n_owners_dev, 
 // step adds the lanes' halves of the values it keeps, so the exchanges halve
 // from step to step (20, 10, 5, 3, 2, 1 for 39 values) where a butterfly per
 // value takes six each. The additions pair lanes 32, 16, 8, 4, 2, 1 apart in
-// this order, as wave_sum does: the totals are its bits.
+// this order, as such a butterfly does.
 template <int M>
 __device__ __forceinline__ void sum_step(float* v, int lane, int n) {
 #pragma unroll
@@ -1634,7 +1627,6 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
   args.grad = a->grad;
   args.node = a->nodeWork;
   args.nNodes = nn;
-  args.entries = E;
   args.tr.start = iw + W.start;
   args.tr.end = iw + W.end;
   args.tr.chunks = iw + W.chunks;
@@ -1714,8 +1706,8 @@ extern "C" int changaGravityAdjoint(const ChangaAdjointLaunch* a, void* stream) 
     CGPU_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     hipLaunchKernelGGL(adj_cells_kernel, dim3(ncu * 16), dim3(kWave), 0, s, args);
     CGPU_CHECK(hipGetLastError());
-    // (records that are not line-aligned are left aside: the wire moments
-    // hold the same values)
+    // (records that are not line-aligned are left aside, not refused: the wire
+    // moments hold the same values)
     const bool rec = args.pc.cellRecords &&
                      reinterpret_cast<uintptr_t>(args.pc.cellRecords) % CHANGA_CELL_RECORD_BYTES == 0;
     const auto targets = pp.listKind == 1

@@ -284,7 +284,9 @@ int changaBatchedGravityNoAlloc(const ChangaGravityLaunch *cells, const ChangaGr
  * its dependence on the root's centre of mass, moments and h-table).
  * ====================================================================== */
 typedef struct {
-  ChangaGravityLaunch cells;      /* particle-cell launch (listKind 0, tpos64 and cm64 set) */
+  ChangaGravityLaunch cells;      /* particle-cell launch (listKind 0, tpos64 and cm64 set); the
+                                     target side reads its cellRecords when they are set and
+                                     128-byte aligned, else the wire moments: the same values */
   ChangaGravityLaunch parts;      /* particle-particle launch (spos64 set), same buckets */
   const float *w;                 /* dL/da, 3 per target, in target order (device) */
   const int *targetIndex;         /* particle index of each target (device), or NULL when the
