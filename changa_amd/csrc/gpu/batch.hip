@@ -230,11 +230,10 @@ namespace {
 // 4,051 114 / 94 / 95, 7,985 174 / 161 / 172, 12,004 603 / 599 / 642, 15,948
 // 314 / 309 / 341, 20,185 of a sparse rung 188 / 199 / 265. The launch is made
 // to have the card to itself. Where it has not, teams cost: 8 plans on 8
-// streams, 1,203 / 1,550 / 1,872 buckets, 305 / 382 / 454 us with four, 229 /
-// 310 / 380 with two, 217 / 268 / 310 with one (a single one 61 / 71 / 77, 59 /
-// 71 / 80, 78 / 86 / 92), so four stop at 1,024, where two are as good; 6,049
-// buckets 1,177 with two and 1,076 with one, where a single one takes 180 and
-// 199, so two stay.
+// streams, 1,203 / 1,550 / 1,872 buckets, 251 / 317 / 380 us with four, 192 /
+// 260 / 323 with two, 188 / 228 / 268 with one (a single plan 53 / 60 / 66, 54
+// / 66 / 72, 69 / 78 / 81), so four stop at 1,024; 6,049 buckets 1,025 with two
+// and 955 with one, a single plan 160 and 173, so two stay.
 int batch_waves(int buckets) { return team_waves(buckets, 1024, 8192); }
 
 // Workgroups of the persistent kernel over this many buckets: those resident

@@ -107,10 +107,12 @@ __device__ __forceinline__ void ewald_term32(const EwaldMom32& Q, float x, float
 // particles near a replica's copy of the root centre) from the exponential
 // the recursion needs anyway: erfc(x) = e^(-x^2) P(t), t = 1 / (1 + x / 2),
 // -erf = erfc - 1. P: degree-7 least-maximum fit of erfc(x) e^(x^2) on
-// 0.98 <= x <= 6.3 (own fit, relative error 1e-8; below that range's end
-// e^(-x^2) is zero to FP32). With e^(-x^2) from the unrounded x^2 the
-// relative error of erfc is at most 3.4e-7 for x <= 6.2, where erfcf of the
-// rounded x gives 6.5e-6, at a third of its instructions.
+// 0.98 <= x <= 6.3 (own fit, relative error 1e-8; 2.2e-7 up to 7, 5.2e-6 up
+// to 9.2, 1e-4 up to 15, where it does not matter: erfc is below 1e-17 past
+// 6.3, far under the sums' FP64 rounding of terms of order one). With
+// e^(-x^2) from the unrounded x^2 the relative error of erfc is at most
+// 3.4e-7 for x <= 6.2, where erfcf of the rounded x gives 6.5e-6, at a third
+// of its instructions.
 __device__ __forceinline__ void radial32_fast(float r2, float hole, float alpha, float alpha2,
                                               float ka, float inner2, float* g) {
   const float dir = rsqrtf(r2), ir2 = dir * dir;

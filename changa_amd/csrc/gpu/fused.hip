@@ -84,9 +84,10 @@ __device__ bool fused_walk(const FusedArgs& a, int b, int lane, unsigned* stack,
   return ok;
 }
 
-// Four wavefronts per SIMD (128 VGPRs, no spills): the walk's load latency is
-// hidden behind more resident wavefronts and the force loops' FP32
-// instructions issue together (gravity_body.h: pc_cells).
+// Four wavefronts per SIMD (128 VGPRs; 12 spilled with records, 7 without,
+// outside the force loops): the walk's load latency is hidden behind more
+// resident wavefronts and the force loops' FP32 instructions issue together
+// (gravity_body.h: pc_cells).
 // REC: cells from the 128-byte cell records (a.pc.cellRecords), whole-line
 // fetches in tiles of PCT.
 template <int PCT, int PPT, bool REC>

@@ -8,16 +8,16 @@
 // nodeGravityComputation / particleGravityComputation (HostCUDA.cu:1008-1205,
 // 1565-1751).
 //
-// Decomposition. One 64-lane wavefront (one workgroup) owns one target
-// bucket: lanes are split into `nslot` slots of `nt` targets (nt = bucket
-// size, nslot = 64 / nt), so a 16-particle bucket keeps 4 source slots busy
-// and an 11-particle bucket 5. Sources are staged through LDS in tiles: the
+// Decomposition. One workgroup owns one target bucket: one 64-lane wavefront,
+// or, in launches of few buckets, two or four that share its lists (Team). A
+// wavefront's lanes are split into `nslot` slots over the `nt` targets, one
+// or more per lane (Lanes). Sources are staged through LDS in tiles: the
 // cells' 27-float records are fetched with coalesced flat loads, pre-scaled
 // (moments times n c_n radius^n, replica offset applied) once per tile, and
 // read back as broadcast ds_read_b128. Each lane accumulates its slot's
 // contributions in FP32 within a tile and folds them into FP64 after each
-// tile; the slots are reduced in a fixed order through LDS, so the result is
-// deterministic. Accelerations and potentials are added into the
+// tile; the slots, and a team's wavefronts after them, are reduced in a fixed
+// order through LDS, so the result is deterministic. Accelerations and potentials are added into the
 // VariablePartData array (+=), dtGrav takes the max.
 #pragma once
 #include <utility>

@@ -74,8 +74,11 @@ void TransferParticleVarsBack(VariablePartData *hostBuffer, size_t size, void *d
    periodic replica, with theta / thetaMono, and gets the PC, softened-cell
    and PP forces of what the walk accepts (+= / max as above), with the
    replica periods fperiod, fperiodY, fperiodZ per axis; a walk beyond the
-   per-wavefront scratch (16,384 cells, 8,192 particle runs) or a child or
-   bucket index outside its array is reported as an error. */
+   scratch of a bucket (16,384 cells, 8,192 particle runs) or a child or
+   bucket index outside its array is reported as an error. The stream's pool
+   holds 224 KiB of scratch per 64 particles of its largest request, at most
+   one per resident wavefront (about 940 MB), 4 bytes a particle, and a
+   quarter of the sum more. */
 void TreePieceCellListDataTransferLocal(CudaRequest *data);
 void TreePieceCellListDataTransferRemote(CudaRequest *data);
 void TreePieceCellListDataTransferRemoteResume(CudaRequest *data);
@@ -371,7 +374,7 @@ int changaBuildListsFill(const ChangaListBuild *b, void *stream);
  * bucketSize particles (Compute.cpp:2476), numbered breadth first; buckets
  * in particle order. The outputs are the topology changaBuildMoments,
  * changaBuildLists* and changaGravityAdjoint take. Synchronizes the stream
- * (one count per depth is read back).
+ * (the depths' node counts are read back, 16 depths at a time).
  * ====================================================================== */
 typedef struct {
   int n;                          /* particles */
