@@ -32,8 +32,8 @@
 // every step gathered 64 records of 64 bytes, and the texture pipe bounded
 // both passes. The union costs more steps (2,069 a wavefront of 64 in the
 // 128^3 box, about 1.6 times one bucket's), the time of a step is the
-// wavefront's own instructions, and 128^3 took 1.41 + 2.02 ms before, 1.24 +
-// 1.54 now. Loading the records of both possible next nodes ahead cost 40
+// wavefront's own instructions, and 128^3 took 1.41 + 2.02 ms before, 1.17 +
+// 1.41 now. Loading the records of both possible next nodes ahead cost 40
 // more scalar instructions a step (1.49 + 1.50), through one vector load and
 // readlanes 1.84 + 1.92. (A wavefront's lanes on the nodes of one bucket,
 // the fused form's walk, measured slower too.)

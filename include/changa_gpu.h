@@ -172,7 +172,7 @@ int changaAddVars(VariablePartData *dst, const VariablePartData *src, int n, voi
 
 /* Ewald on device-resident data. markers: n active particle indices into
    parts (device memory; NULL: particles first..first+n-1). ewt: the
-   ro->nEwhLoop table entries in device memory. ro: host struct (its
+   ro->nEwhLoop table entries (at most 4,348) in device memory. ro: host struct (its
    momcRoot, mm, L, fEwCut, nReps and nEwReps are used). Precision form:
    pos64 (device, 3 per particle) and rootCm64 (host, 3 doubles) or NULL. */
 int changaEwald(const CompactPartData *parts, VariablePartData *vars, const int *markers,
